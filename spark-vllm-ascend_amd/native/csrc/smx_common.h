@@ -48,11 +48,26 @@ __device__ __forceinline__ void st_agent(u32x4* p, u32x4 v) {  // two 64-bit sto
   st_agent(q, (uint64_t)v.x | ((uint64_t)v.y << 32));
   st_agent(q + 1, (uint64_t)v.z | ((uint64_t)v.w << 32));
 }
+// The same for 16 bytes per lane in ONE store (st_agent on a u32x4 is two
+// 64-bit atomic stores, each of which writes half of every 16 bytes through):
+// a raw buffer store with the sc1 cache policy, at byte offset off from the
+// wave-uniform base of r.  Lanes at or past r's byte count store nothing.
+// The kernels that stream megabytes (dequantisation, the element-wise ops of
+// a prefill chunk) store this way.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t agent_rsrc(void* base, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00027000);
+}
+__device__ __forceinline__ void st_agent_b128(__amdgpu_buffer_rsrc_t r, uint32_t off, u32x4 v) {
+  constexpr int SC1 = 16;  // cache-policy bit of gfx940 and later
+  __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, SC1);
+}
 __device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0); }
 
 // Unaligned-to-16 (but 4-byte aligned) vector types for the Q4_0 stream:
 // GGUF blocks are 18 bytes, so a block pair starts on a 4-byte boundary only.
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
+typedef u32x4 u32x4_a2 __attribute__((aligned(2)));  // one block of a row of any K % 32
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t h16) {
   return __uint_as_float(h16 << 16);

@@ -55,6 +55,23 @@ def test_dequant_bit_exact(ops, dev, n, k):
     np.testing.assert_array_equal(got, ref)
 
 
+@pytest.mark.parametrize("n", [1, 63, 255, 256, 257, 511])
+@pytest.mark.parametrize("shift", [0, 2])
+def test_dequant_workgroup_edges_and_alignment(ops, dev, n, shift):
+    """Block counts around a workgroup's 256, weights 2-byte and outputs
+    4-byte aligned: bit-exact, and nothing past the last block is written."""
+    import torch
+    k = 32
+    blocks = oq.make_blocks(n, k, seed=700 + n)
+    w = torch.empty(n * 18 + shift, dtype=torch.uint8, device=dev)
+    w[shift:] = _blocks_dev(blocks, dev).view(-1)
+    buf = torch.full((shift + n * k + 512,), -7.0, dtype=torch.bfloat16, device=dev)
+    ops.q4_0_dequant_bf16(w[shift:], n, k, out=buf[shift:shift + n * k])
+    np.testing.assert_array_equal(bits_of(buf[shift:shift + n * k]).reshape(n, k),
+                                  oq.c_dequant_bf16_bits(blocks, n, k))
+    assert bool((buf[:shift] == -7.0).all()) and bool((buf[shift + n * k:] == -7.0).all())
+
+
 def test_dequant_special_scales(ops, dev):
     blocks, n, k = _kat_blocks()
     got = bits_of(ops.q4_0_dequant_bf16(_blocks_dev(blocks, dev), n, k)).reshape(n, k)
