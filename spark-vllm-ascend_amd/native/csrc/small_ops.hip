@@ -79,10 +79,10 @@ __global__ __launch_bounds__(1024) void add_rmsnorm_kernel(
         ro[i] = pack_bf16x2(s0, s1);
         yo[i] = pack_bf16x2(s0 * inv * bf16_lo(gw[i]), s1 * inv * bf16_hi(gw[i]));
       }
-      st_agent(reinterpret_cast<u32x4*>(y + row * hidden) + ch, u32x4{yo[0], yo[1], yo[2], yo[3]});
+      st_agent_b128(reinterpret_cast<u32x4*>(y + row * hidden) + ch, u32x4{yo[0], yo[1], yo[2], yo[3]});
       if (residual_out)
-        st_agent(reinterpret_cast<u32x4*>(residual_out + row * hidden) + ch,
-                 u32x4{ro[0], ro[1], ro[2], ro[3]});
+        st_agent_b128(reinterpret_cast<u32x4*>(residual_out + row * hidden) + ch,
+                      u32x4{ro[0], ro[1], ro[2], ro[3]});
     }
   }
   stores_done();
@@ -142,6 +142,78 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_kernel(
   stores_done();
 }
 
+// The same with 16-byte accesses (every tensor 16-byte aligned): 16 lanes per
+// head, lane j dims 8 j .. 8 j + 7, four consecutive (token, head) pairs per
+// wave.  Bound by memory; a wave per head with 2-byte accesses moved a
+// prefill chunk of 2047 tokens x 48 heads in 25.9 us, this in 13.6 (50 MB).  Lane j ^ 8
+// holds the other half of each rotation pair and the squares are summed in
+// the one-wave kernel's order, so both kernels round alike.
+__global__ __launch_bounds__(256) void qknorm_rope_kv_vec_kernel(
+    const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ q_gamma,
+    const uint16_t* __restrict__ k_gamma, const uint16_t* __restrict__ cos_sin,
+    const int64_t* __restrict__ positions, const int64_t* __restrict__ slot_mapping,
+    uint16_t* __restrict__ q_out, uint16_t* __restrict__ k_cache, uint16_t* __restrict__ v_cache,
+    uint32_t items, int n_q, int n_kv, int64_t cache_slots, int max_position, float eps) {
+  constexpr int HD = 128, HALF = 64;
+  const int j = threadIdx.x & 15, dim = 8 * (j & 7);
+  const uint32_t raw = blockIdx.x * 16u + (threadIdx.x >> 4);
+  // lanes past the end work on the last item (the row moves below need every
+  // lane) and store nothing
+  const uint32_t item = min(raw, items - 1);
+  const uint32_t nh = (uint32_t)(n_q + 2 * n_kv);
+  const uint32_t t = item / nh;
+  const int h = (int)(item - t * nh);
+  const u32x4 own = *reinterpret_cast<const u32x4*>(qkv + (int64_t)item * HD + 8 * j);
+  const int64_t slot = slot_mapping[t];
+  int64_t pos = positions[t];
+  const uint16_t* gam = h < n_q ? q_gamma : k_gamma;
+  const u32x4 gv = *reinterpret_cast<const u32x4*>(gam + 8 * j);
+  pos = pos < 0 ? 0 : (pos >= max_position ? max_position - 1 : pos);
+  const u32x4 cv = *reinterpret_cast<const u32x4*>(cos_sin + pos * HD + dim);
+  const u32x4 sv = *reinterpret_cast<const u32x4*>(cos_sin + pos * HD + HALF + dim);
+  auto other_half = [](uint32_t v) {  // lane j ^ 8's register
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, DPP_ROW_ROR8, 0xf, 0xf, false);
+  };
+  u32x4 val = own;
+  // (every head of a wave is a V head, or all lanes stay: the row moves need them)
+  if (__builtin_amdgcn_ballot_w64(h < n_q + n_kv) != 0) {
+    const bool lo = j < 8;
+    float sq[8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t p = other_half(own[i]);
+      const uint32_t aw = lo ? own[i] : p, bw = lo ? p : own[i];
+      sq[2 * i] = bf16_lo(aw) * bf16_lo(aw) + bf16_lo(bw) * bf16_lo(bw);
+      sq[2 * i + 1] = bf16_hi(aw) * bf16_hi(aw) + bf16_hi(bw) * bf16_hi(bw);
+    }
+    const float ss = sum8(((sq[0] + sq[1]) + (sq[2] + sq[3])) + ((sq[4] + sq[5]) + (sq[6] + sq[7])));
+    const float inv = 1.0f / sqrtf(ss / (float)HD + eps);
+    const uint32_t flip = lo ? 0x80008000u : 0u;  // u = a c - b s, v = b c + a s
+    uint32_t r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // the rounded norm of this half, and the other half's from lane j ^ 8
+      const uint32_t nw = pack_bf16x2(bf16_lo(own[i]) * inv * bf16_lo(gv[i]),
+                                      bf16_hi(own[i]) * inv * bf16_hi(gv[i]));
+      const uint32_t ow = other_half(nw), sw = sv[i] ^ flip;
+      r[i] = pack_bf16x2(fmaf(bf16_lo(nw), bf16_lo(cv[i]), bf16_lo(ow) * bf16_lo(sw)),
+                         fmaf(bf16_hi(nw), bf16_hi(cv[i]), bf16_hi(ow) * bf16_hi(sw)));
+    }
+    if (h < n_q + n_kv) val = u32x4{r[0], r[1], r[2], r[3]};
+  }
+  const bool write_kv = slot >= 0 && slot < cache_slots;
+  uint16_t* dst;
+  if (h < n_q) {
+    dst = q_out + ((int64_t)t * n_q + h) * HD;
+  } else if (h < n_q + n_kv) {
+    dst = k_cache + (slot * n_kv + (h - n_q)) * HD;
+  } else {
+    dst = v_cache + (slot * n_kv + (h - n_q - n_kv)) * HD;
+  }
+  if (raw < items && (h < n_q || write_kv)) st_agent_b128(dst + 8 * j, val);
+  stores_done();
+}
+
 // out = bf16(silu(g) * u) with silu(g) = g / (1 + exp(-g)), all in fp32.
 __global__ __launch_bounds__(256) void silu_mul_kernel(const uint16_t* __restrict__ gu,
                                                        uint16_t* __restrict__ out, int64_t rows,
@@ -167,6 +239,74 @@ __global__ __launch_bounds__(256) void gelu_mul_kernel(const uint16_t* __restric
   const uint16_t g = gu[r * 2 * d + c];
   const float u = bf16_bits_to_f32(gu[r * 2 * d + d + c]);
   st_agent(out + i, f32_to_bf16(bf16_bits_to_f32(gelu_lut(g, lut)) * u));
+  stores_done();
+}
+
+// The two gated activations with 16-byte accesses (d a multiple of 8, both
+// tensors 16-byte aligned): each thread takes ITERS chunks of 8 outputs, all
+// loads first.  Bound by memory: one element a thread, with a 64-bit
+// division and a 2-byte store each, took 48.4 us for 2047 x 9728 (120 MB);
+// this takes 24.0.  GELU looks its table up in LDS.
+template <bool GELU, int ITERS>
+__global__ __launch_bounds__(256) void gated_mul_vec_kernel(
+    const uint16_t* __restrict__ gu, const uint16_t* __restrict__ lut, uint16_t* __restrict__ out,
+    uint32_t total, uint32_t nch) {
+  __shared__ __attribute__((aligned(16))) uint16_t tab[GELU ? kGeluLutEntries : 8];
+  const uint32_t c0 = blockIdx.x * (256u * ITERS);  // first output chunk
+  const u32x4* src = reinterpret_cast<const u32x4*>(gu);
+  u32x4 g[ITERS], u[ITERS];
+#pragma unroll
+  for (int k = 0; k < ITERS; ++k) {
+    const uint32_t i = min(c0 + 256u * k + threadIdx.x, total - 1);
+    const uint32_t r = i / nch;
+    const u32x4* p = src + (int64_t)i + (int64_t)r * nch;  // row r starts at 2 r nch
+    g[k] = p[0];
+    u[k] = p[nch];
+  }
+  if constexpr (GELU) {
+    for (int i = threadIdx.x; i < kGeluLutEntries; i += 256) tab[i] = lut[i];
+    __syncthreads();
+  }
+  const auto rsrc = agent_rsrc(out + (int64_t)c0 * 8, min(256u * ITERS, total - c0) * 16u);
+#pragma unroll
+  for (int k = 0; k < ITERS; ++k) {
+    uint32_t o[4];
+#pragma unroll
+    for (int w = 0; w < 4; ++w) {
+      float y[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const float uv = e ? bf16_hi(u[k][w]) : bf16_lo(u[k][w]);
+        if constexpr (GELU) {
+          const uint32_t gb = (g[k][w] >> (16 * e)) & 0xffffu;
+          y[e] = bf16_bits_to_f32(gelu_lut(gb, tab)) * uv;
+        } else {
+          const float gv = e ? bf16_hi(g[k][w]) : bf16_lo(g[k][w]);
+          y[e] = gv / (1.0f + expf(-gv)) * uv;
+        }
+      }
+      o[w] = pack_bf16x2(y[0], y[1]);
+    }
+    // chunks past the end are dropped by the resource's bounds
+    st_agent_b128(rsrc, (256u * k + threadIdx.x) * 16u, u32x4{o[0], o[1], o[2], o[3]});
+  }
+  stores_done();
+}
+
+// Rows of a bf16 table with 16-byte accesses (hidden a multiple of 8, both
+// tensors 16-byte aligned); grid (gx, tokens), nt threads of one chunk each.
+__global__ __launch_bounds__(256) void embedding_vec_kernel(const uint16_t* __restrict__ table,
+                                                            const int64_t* __restrict__ ids,
+                                                            uint16_t* __restrict__ out,
+                                                            int64_t vocab, int nch, int nt) {
+  const int64_t t = blockIdx.y;
+  const int64_t id = ids[t];
+  const bool ok = id >= 0 && id < vocab;
+  const int c = (int)blockIdx.x * nt + (int)threadIdx.x;
+  if (c < nch) {
+    const u32x4 v = reinterpret_cast<const u32x4*>(table)[(ok ? id : 0) * nch + c];
+    st_agent_b128(reinterpret_cast<u32x4*>(out) + t * nch + c, ok ? v : u32x4{0u, 0u, 0u, 0u});
+  }
   stores_done();
 }
 
@@ -367,6 +507,25 @@ __global__ __launch_bounds__(64) void reshape_and_cache_kernel(
   stores_done();
 }
 
+// The same with 16-byte accesses (head_dim a multiple of 8, every tensor
+// 16-byte aligned): a token's n_kv heads are contiguous on both sides, so one
+// workgroup of nt threads copies its K row of nch chunks, then its V row.
+__global__ __launch_bounds__(256) void reshape_and_cache_vec_kernel(
+    const u32x4* __restrict__ key, const u32x4* __restrict__ value, u32x4* __restrict__ k_cache,
+    u32x4* __restrict__ v_cache, const int64_t* __restrict__ slot_mapping, int nch,
+    int64_t cache_slots, int nt) {
+  const int64_t t = blockIdx.x;
+  const int64_t slot = slot_mapping[t];
+  if (slot < 0 || slot >= cache_slots) return;
+  for (int c = threadIdx.x; c < 2 * nch; c += nt) {
+    const bool k = c < nch;
+    const int o = k ? c : c - nch;
+    const u32x4 v = (k ? key : value)[t * nch + o];
+    st_agent_b128((k ? k_cache : v_cache) + slot * nch + o, v);
+  }
+  stores_done();
+}
+
 // Slot of every token of a (ragged) batch: token t of request r (the r with
 // query_start_loc[r] <= t < query_start_loc[r + 1]) at position p goes to
 // block_table[r][p / block_size] * block_size + p % block_size; tokens in no
@@ -401,6 +560,14 @@ __global__ __launch_bounds__(256) void slot_mapping_kernel(
 }  // namespace smx
 
 #include "smx_abi_util.h"
+
+namespace {
+// Whether every pointer allows 16-byte accesses.
+template <typename... P>
+bool aligned16(const P*... p) {
+  return (... && ((uintptr_t)p % 16 == 0));
+}
+}  // namespace
 
 extern "C" int smx_add_rmsnorm(void* stream, const void* x, const void* residual,
                                const void* gamma, void* y, void* residual_out, int64_t rows,
@@ -444,6 +611,15 @@ extern "C" int smx_qknorm_rope_kv_write(void* stream, const void* qkv, const voi
   SMX_REQUIRE(eps >= 0.f && isfinite(eps), "eps must be finite and >= 0");
   SMX_REQUIRE((uintptr_t)positions % 8 == 0 && (uintptr_t)slot_mapping % 8 == 0,
               "int64 arrays must be 8-byte aligned");
+  if (aligned16(qkv, q_gamma, k_gamma, cos_sin, q_out, k_cache, v_cache)) {
+    const uint32_t items = (uint32_t)num_tokens * (uint32_t)(n_q + 2 * n_kv);  // <= 65535^2
+    SMX_LAUNCH(smx::qknorm_rope_kv_vec_kernel, dim3(items / 16 + (items % 16 != 0)), dim3(256), 0,
+               (hipStream_t)stream, (const uint16_t*)qkv, (const uint16_t*)q_gamma,
+               (const uint16_t*)k_gamma, (const uint16_t*)cos_sin, positions, slot_mapping,
+               (uint16_t*)q_out, (uint16_t*)k_cache, (uint16_t*)v_cache, items, n_q, n_kv,
+               (int64_t)num_blocks * block_size, max_position, eps);
+    return (int)hipGetLastError();
+  }
   SMX_LAUNCH(smx::qknorm_rope_kv_kernel, dim3(n_q + 2 * n_kv, num_tokens), dim3(64), 0,
                      (hipStream_t)stream, (const uint16_t*)qkv, (const uint16_t*)q_gamma,
                      (const uint16_t*)k_gamma, (const uint16_t*)cos_sin, positions, slot_mapping,
@@ -452,12 +628,29 @@ extern "C" int smx_qknorm_rope_kv_write(void* stream, const void* qkv, const voi
   return (int)hipGetLastError();
 }
 
+namespace {
+template <bool GELU>
+int launch_gated_vec(void* stream, const void* gate_up, const void* lut, void* out, int64_t rows,
+                     int64_t d) {
+  const uint32_t nch = (uint32_t)(d / 8), total = (uint32_t)rows * nch;  // < 2^31
+  // one chunk a thread while that gives at most 4 workgroups per CU, then four
+  const bool few = total <= 1024u * 256u;
+  const uint32_t per = few ? 256u : 1024u;
+  SMX_LAUNCH((few ? smx::gated_mul_vec_kernel<GELU, 1> : smx::gated_mul_vec_kernel<GELU, 4>),
+             dim3((total + per - 1) / per), dim3(256), 0, (hipStream_t)stream,
+             (const uint16_t*)gate_up, (const uint16_t*)lut, (uint16_t*)out, total, nch);
+  return (int)hipGetLastError();
+}
+}  // namespace
+
 extern "C" int smx_silu_mul(void* stream, const void* gate_up, void* out, int64_t rows,
                             int64_t d) {
   SMX_REQUIRE(gate_up && out, "null pointer argument");
   SMX_REQUIRE(rows >= 1 && d >= 1 && rows * d < (1ll << 40), "bad shape");
   const int64_t grid = (rows * d + 255) / 256;
   SMX_REQUIRE(grid < (1ll << 31), "tensor too large");
+  if (d % 8 == 0 && rows * d < (1ll << 34) && aligned16(gate_up, out))
+    return launch_gated_vec<false>(stream, gate_up, nullptr, out, rows, d);
   SMX_LAUNCH(smx::silu_mul_kernel, dim3((unsigned)grid), dim3(256), 0,
                      (hipStream_t)stream, (const uint16_t*)gate_up, (uint16_t*)out, rows, d);
   return (int)hipGetLastError();
@@ -471,6 +664,8 @@ extern "C" int smx_gelu_mul(void* stream, const void* gate_up, const void* lut, 
   SMX_REQUIRE(rows >= 1 && d >= 1 && rows * d < (1ll << 40), "bad shape");
   const int64_t grid = (rows * d + 255) / 256;
   SMX_REQUIRE(grid < (1ll << 31), "tensor too large");
+  if (d % 8 == 0 && rows * d < (1ll << 34) && aligned16(gate_up, out))
+    return launch_gated_vec<true>(stream, gate_up, lut, out, rows, d);
   SMX_LAUNCH(smx::gelu_mul_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream,
              (const uint16_t*)gate_up, (const uint16_t*)lut, (uint16_t*)out, rows, d);
   return (int)hipGetLastError();
@@ -482,6 +677,13 @@ extern "C" int smx_embedding(void* stream, const void* table, const int64_t* ids
   SMX_REQUIRE(num_tokens >= 1 && num_tokens <= 65535, "num_tokens must be in [1, 65535]");
   SMX_REQUIRE(vocab >= 1 && hidden >= 1, "vocab and hidden must be >= 1");
   SMX_REQUIRE((uintptr_t)ids % 8 == 0, "ids must be 8-byte aligned");
+  if (hidden % 8 == 0 && hidden <= (1 << 24) && aligned16(table, out)) {
+    const int nch = (int)(hidden / 8), gxv = (nch + 255) / 256;
+    const int nt = ((nch + gxv - 1) / gxv + 63) / 64 * 64;
+    SMX_LAUNCH(smx::embedding_vec_kernel, dim3(gxv, (unsigned)num_tokens), dim3(nt), 0,
+               (hipStream_t)stream, (const uint16_t*)table, ids, (uint16_t*)out, vocab, nch, nt);
+    return (int)hipGetLastError();
+  }
   const unsigned gx = (unsigned)((hidden + 255) / 256 < 64 ? (hidden + 255) / 256 : 64);
   SMX_LAUNCH(smx::embedding_kernel, dim3(gx, (unsigned)num_tokens), dim3(256), 0,
                      (hipStream_t)stream, (const uint16_t*)table, ids, (uint16_t*)out, vocab,
@@ -508,6 +710,15 @@ extern "C" int smx_reshape_and_cache(void* stream, const void* key, const void* 
   SMX_REQUIRE(n_kv >= 1 && n_kv <= 65535 && head_dim >= 1 && head_dim <= 4096, "bad head shape");
   SMX_REQUIRE(num_blocks >= 1 && block_size >= 1, "num_blocks and block_size must be >= 1");
   SMX_REQUIRE((uintptr_t)slot_mapping % 8 == 0, "slot_mapping must be 8-byte aligned");
+  const int64_t row = (int64_t)n_kv * head_dim;  // < 2^29
+  if (head_dim % 8 == 0 && aligned16(key, value, k_cache, v_cache)) {
+    const int nch = (int)(row / 8), nt = nch >= 128 ? 256 : (2 * nch + 63) / 64 * 64;
+    SMX_LAUNCH(smx::reshape_and_cache_vec_kernel, dim3(num_tokens), dim3(nt), 0,
+               (hipStream_t)stream, (const smx::u32x4*)key, (const smx::u32x4*)value,
+               (smx::u32x4*)k_cache, (smx::u32x4*)v_cache, slot_mapping, nch,
+               (int64_t)num_blocks * block_size, nt);
+    return (int)hipGetLastError();
+  }
   SMX_LAUNCH(smx::reshape_and_cache_kernel, dim3(n_kv, num_tokens), dim3(64), 0,
                      (hipStream_t)stream, (const uint16_t*)key, (const uint16_t*)value,
                      (uint16_t*)k_cache, (uint16_t*)v_cache, slot_mapping, n_kv, head_dim,

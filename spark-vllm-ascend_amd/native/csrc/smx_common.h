@@ -49,17 +49,24 @@ __device__ __forceinline__ void st_agent(u32x4* p, u32x4 v) {  // two 64-bit sto
   st_agent(q + 1, (uint64_t)v.z | ((uint64_t)v.w << 32));
 }
 // The same for 16 bytes per lane in ONE store (st_agent on a u32x4 is two
-// 64-bit atomic stores, each of which writes half of every 16 bytes through):
-// a raw buffer store with the sc1 cache policy, at byte offset off from the
-// wave-uniform base of r.  Lanes at or past r's byte count store nothing.
+// 64-bit atomic stores, each of which writes half of every 16 bytes through).
 // The kernels that stream megabytes (dequantisation, the element-wise ops of
-// a prefill chunk) store this way.
+// a prefill chunk) store this way:
+//  * agent_rsrc + st_agent_b128(r, off, v): a raw buffer store with the sc1
+//    cache policy, at byte offset off from the wave-uniform base of r; lanes
+//    at or past r's byte count store nothing;
+//  * st_agent_b128(p, v): any 16-byte aligned address per lane.  The s_nop is
+//    the wait state a store of more than 64 bits needs before its data
+//    registers are overwritten, which the compiler does not add after an asm.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t agent_rsrc(void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00027000);
 }
 __device__ __forceinline__ void st_agent_b128(__amdgpu_buffer_rsrc_t r, uint32_t off, u32x4 v) {
   constexpr int SC1 = 16;  // cache-policy bit of gfx940 and later
   __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, SC1);
+}
+__device__ __forceinline__ void st_agent_b128(void* p, u32x4 v) {
+  __asm__ volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
 }
 __device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0); }
 
@@ -147,6 +154,7 @@ constexpr int DPP_QUAD_XOR1 = 0xB1;      // quad_perm [1,0,3,2]
 constexpr int DPP_QUAD_XOR2 = 0x4E;      // quad_perm [2,3,0,1]
 constexpr int DPP_ROW_HALF_MIRROR = 0x141;
 constexpr int DPP_ROW_MIRROR = 0x140;
+constexpr int DPP_ROW_ROR8 = 0x128;      // lane j of a row gets lane j ^ 8
 
 // Sum over each aligned group of 8 lanes; every lane of the group gets it.
 __device__ __forceinline__ float sum8(float v) {

@@ -94,6 +94,77 @@ def test_silu_mul(ops, dev, rows, d):
     assert bf16_ulp_diff(bits_of(out).reshape(rows, d), f32_to_bf16_bits(ref)).max() <= 1
 
 
+def _off(t, shift):
+    """t's values in a contiguous view that starts `shift` elements into its
+    buffer: an odd shift rules 16-byte accesses out."""
+    import torch
+    buf = torch.empty(t.numel() + shift, dtype=t.dtype, device=t.device)
+    buf[shift:] = t.reshape(-1)
+    return buf[shift:].view(t.shape)
+
+
+@pytest.mark.parametrize("rows,d", [(1, 8), (3, 40), (63, 2056), (2, 9728), (257, 8200)])
+@pytest.mark.parametrize("act", ["silu", "gelu"])
+def test_gated_vector_kernel_equals_scalar(ops, dev, rows, d, act):
+    """16-byte and element-wise kernels, bit for bit: sizes around a
+    workgroup's chunks, one and four chunks a thread; nothing past the end."""
+    import torch
+    gu = torch.randn(rows, 2 * d, device=dev).mul_(4).to(torch.bfloat16)
+    gu[0, 0], gu[-1, d - 1] = float("inf"), float("-inf")
+    lut = ops.gelu_table(dev)
+    f = (lambda x, o: ops.silu_mul(x, out=o)) if act == "silu" else (
+        lambda x, o: ops.gelu_mul(x, lut, out=o))
+    buf = torch.full((rows * d + 64,), -7.0, dtype=torch.bfloat16, device=dev)
+    got = f(gu, buf[:rows * d])
+    ref = f(_off(gu, 1), torch.empty(rows, d, dtype=torch.bfloat16, device=dev))
+    np.testing.assert_array_equal(bits_of(got).reshape(-1), bits_of(ref).reshape(-1))
+    assert bool((buf[rows * d:] == -7.0).all())
+
+
+@pytest.mark.parametrize("T,n_q,n_kv", [(1, 4, 1), (5, 3, 1), (17, 32, 8), (3, 8, 2)])
+def test_qknorm_vector_kernel_equals_scalar(ops, dev, T, n_q, n_kv):
+    """The 16-lanes-a-head kernel against the wave-a-head one, bit for bit,
+    with head counts that leave a partial wave and slots that are skipped."""
+    import torch
+    torch.manual_seed(T)
+    nh = n_q + 2 * n_kv
+    qkv = torch.randn(T, nh * 128, device=dev).to(torch.bfloat16)
+    qg, kg = ((1 + 0.1 * torch.randn(128, device=dev)).to(torch.bfloat16) for _ in range(2))
+    cs = torch.randn(64, 128, device=dev).to(torch.bfloat16)
+    pos = torch.randint(-2, 70, (T,), device=dev)  # clamped to the table
+    slots = torch.randperm(96, device=dev)[:T].clone()
+    slots[T // 2] = -1 if T > 1 else slots[0]
+    res = []
+    for shift in (0, 1):
+        kv = torch.zeros(2, 3, 32, n_kv, 128, dtype=torch.bfloat16, device=dev)
+        q = ops.qknorm_rope_kv_write(_off(qkv, shift), qg, kg, cs, pos, slots, kv[0], kv[1], n_q,
+                                     n_kv, 1e-6)
+        res.append((bits_of(q), bits_of(kv)))
+    np.testing.assert_array_equal(res[0][0], res[1][0])
+    np.testing.assert_array_equal(res[0][1], res[1][1])
+
+
+@pytest.mark.parametrize("hidden", [8, 264, 2560, 2056, 4104])
+def test_embedding_and_cache_vector_kernels(ops, dev, hidden):
+    """Gathers and KV copies with 16-byte accesses equal torch's, and the
+    element-wise kernels' (misaligned tensors)."""
+    import torch
+    table = torch.randn(37, hidden, device=dev).to(torch.bfloat16)
+    ids = torch.tensor([36, 0, -1, 5, 37], device=dev)
+    ref = table[ids.clamp(0, 36)] * ((ids >= 0) & (ids < 37)).to(torch.bfloat16)[:, None]
+    slots = torch.tensor([9, -1, 0, 64, 31], device=dev)  # 64: past the cache
+    key, val = (torch.randn(5, 2, hidden // 2, device=dev).to(torch.bfloat16) for _ in range(2))
+    for shift in (0, 1):
+        out = ops.embedding(_off(table, shift), ids)
+        assert torch.equal(out.view(5, hidden), ref.abs() * ref.sign())
+        kv = torch.zeros(2, 2, 32, 2, hidden // 2, dtype=torch.bfloat16, device=dev)
+        ops.reshape_and_cache(_off(key, shift), _off(val, shift), kv[0], kv[1], slots)
+        exp = torch.zeros_like(kv).view(2, 64, 2, hidden // 2)
+        for t in (0, 2, 4):
+            exp[0, slots[t]], exp[1, slots[t]] = key[t], val[t]
+        assert torch.equal(kv.view_as(exp), exp)
+
+
 def test_embedding(ops, dev):
     import torch
     rng = np.random.default_rng(7)
