@@ -323,85 +323,114 @@ __global__ __launch_bounds__(256) void embedding_kernel(const uint16_t* __restri
   stores_done();
 }
 
-// (value, index) ordering for argmax: larger value wins, NaN is largest,
-// ties go to the lower index.
-__device__ __forceinline__ bool better(float v, int64_t i, float bv, int64_t bi) {
-  const bool vn = v != v, bn = bv != bv;
-  if (vn != bn) return vn;
-  if (!vn && v != bv) return v > bv;
-  return i < bi;
+// Order-preserving signed 16-bit keys of bf16 pairs (larger value, larger key;
+// -0 and +0 equal; NaN not ordered): the magnitude, negated for negative values.
+typedef int16_t s16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ s16x2 value_keys(uint32_t w) {
+  const s16x2 s = __builtin_bit_cast(s16x2, w) >> 15;
+  return (__builtin_bit_cast(s16x2, w & 0x7fff7fffu) ^ s) - s;
+}
+// The same for one value, with every NaN above +inf.
+__device__ __forceinline__ int value_key(uint32_t h16) {
+  const int mag = (int)(h16 & 0x7fffu);
+  return mag > 0x7f80 ? 0x7fff : (h16 & 0x8000u) ? -mag : mag;
 }
 
-// One 1024-thread workgroup per row.
+// Greedy argmax, one 1024-thread workgroup per row: the largest value, NaN
+// above all, the lowest index among equal ones.  A row is 300 KB at vocab
+// 151936 and one CU reads it, so what counts is the work per element: a first
+// scan keeps packed 16-bit maxima, 3 VALU operations an element, over 16-byte
+// chunks with AU of them in flight, and notes the group of chunks where the
+// thread's maximum first rose to its value; then the threads that hold the row's
+// maximum look for its index in their group alone.  (Comparing (value, 64-bit
+// index) pairs element by element was bound by one CU's VALU: 25.3 us
+// there, now 11.6.)
+// The elements before the first 16-byte boundary and after the last chunk are
+// one per thread.  A NaN anywhere in the row sends it through an
+// element-by-element scan of the keys that order NaN.
 __global__ __launch_bounds__(1024) void argmax_kernel(const uint16_t* __restrict__ logits,
                                                       int64_t vocab, int64_t* __restrict__ out) {
-  constexpr int64_t NT = 1024;  // threads per workgroup
-  __shared__ float sv[16];
-  __shared__ int64_t si[16];
-  const int64_t row = blockIdx.x;
-  const uint16_t* lr = logits + row * vocab;
-  float bv = -INFINITY;
-  int64_t bi = INT64_MAX;
-  // `better` is a total order, so the scan order does not matter: 16-byte
-  // chunks of 8 values, 4 chunks in flight per thread (a row is 300 KB at
-  // vocab 151936), then the elements the chunks do not cover one by one.
-  int64_t done = 0;
-  if (((uintptr_t)lr & 15) == 0) {
-    const int64_t nch = vocab >> 3;
-    const u32x4* lc = reinterpret_cast<const u32x4*>(lr);
-    for (int64_t c0 = threadIdx.x; c0 < nch; c0 += 4 * NT) {
-      u32x4 v[4];
+  constexpr int NT = 1024;  // threads per workgroup
+  constexpr int AU = 8;     // chunks per thread and group
+  __shared__ int sk[NT / 64], sm[NT / 64];
+  __shared__ int64_t si[NT / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const uint16_t* lr = logits + (int64_t)blockIdx.x * vocab;
+  const int64_t head = min(vocab, (int64_t)(((0 - (uintptr_t)lr) & 15) >> 1));
+  const int64_t nch = (vocab - head) >> 3;
+  const int64_t tail = head + 8 * nch;
+  const u32x4* lc = reinterpret_cast<const u32x4*>(lr + head);
+  // this thread's element outside the chunks (at most 7 before and 7 after)
+  const int64_t lone = tid < head ? tid : tail + (tid - head) < vocab ? tail + (tid - head) : -1;
+
+  int best = lone >= 0 ? value_key(lr[lone]) : -0x8000;
+  int64_t grp = -1;  // first chunk of the group `best` comes from (-1: the lone element)
+  s16x2 mag = s16x2{0, 0};
+  for (int64_t c0 = tid; c0 < nch; c0 += AU * NT) {
+    u32x4 v[AU];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t c = c0 + u * NT;
-        v[u] = lc[c < nch ? c : nch - 1];
-      }
+    for (int u = 0; u < AU; ++u) v[u] = lc[min(c0 + (int64_t)u * NT, nch - 1)];
+    s16x2 mx = s16x2{-0x8000, -0x8000};
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int64_t c = c0 + u * NT;
-        if (c >= nch) continue;
-        const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+    for (int u = 0; u < AU; ++u) {
+      const uint32_t w[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = (e & 1) ? bf16_hi(w[e >> 1]) : bf16_lo(w[e >> 1]);
-          if (better(x, c * 8 + e, bv, bi)) {
-            bv = x;
-            bi = c * 8 + e;
-          }
-        }
+      for (int e = 0; e < 4; ++e) {
+        mx = __builtin_elementwise_max(mx, value_keys(w[e]));
+        mag = __builtin_elementwise_max(mag, __builtin_bit_cast(s16x2, w[e] & 0x7fff7fffu));
       }
     }
-    done = nch << 3;
-  }
-  for (int64_t i = done + threadIdx.x; i < vocab; i += NT) {
-    const float v = bf16_bits_to_f32(lr[i]);
-    if (better(v, i, bv, bi)) {
-      bv = v;
-      bi = i;
+    const int k = max((int)mx.x, (int)mx.y);
+    if (k > best) {
+      best = k;
+      grp = c0;
     }
   }
-  // wave reduction with shuffles
-  for (int m = 32; m >= 1; m >>= 1) {
-    const float ov = __shfl_xor(bv, m, 64);
-    const int64_t oi = __shfl_xor(bi, m, 64);
-    if (better(ov, oi, bv, bi)) {
-      bv = ov;
-      bi = oi;
-    }
+  // the row's maximum, and whether any element is NaN
+  int m = max(best, 0) > 0x7f80 ? 0x7fff : max((int)mag.x, (int)mag.y), mk = best;
+  for (int o = 32; o >= 1; o >>= 1) {
+    mk = max(mk, __shfl_xor(mk, o, 64));
+    m = max(m, __shfl_xor(m, o, 64));
   }
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) {
-    sv[wave] = bv;
-    si[wave] = bi;
+    sk[wave] = mk;
+    sm[wave] = m;
   }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int wv = 1; wv < (int)(NT >> 6); ++wv)
-      if (better(sv[wv], si[wv], bv, bi)) {
-        bv = sv[wv];
-        bi = si[wv];
-      }
-    st_agent(out + row, bi == INT64_MAX ? (int64_t)0 : bi);
+#pragma unroll
+  for (int i = 0; i < NT / 64; ++i) {
+    mk = max(mk, sk[i]);
+    m = max(m, sm[i]);
+  }
+  int64_t idx = INT64_MAX;
+  auto look = [&](int64_t c0, int want) {  // lowest element of the group with key `want`
+#pragma unroll 1
+    for (int u = 0; u < AU; ++u) {
+      const int64_t c = c0 + (int64_t)u * NT;
+      if (c >= nch) break;
+      const u32x4 v = lc[c];
+      const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (value_key(e & 1 ? w[e >> 1] >> 16 : w[e >> 1] & 0xffffu) == want)
+          idx = min(idx, head + 8 * c + e);
+    }
+  };
+  if (m > 0x7f80) {  // uniform: some element is NaN, and the first one wins
+    if (lone >= 0 && value_key(lr[lone]) == 0x7fff) idx = lone;
+    for (int64_t c0 = tid; c0 < nch; c0 += AU * NT) look(c0, 0x7fff);
+  } else if (best == mk) {
+    // (a chunk value equal to the lone element's does not set grp: look at both)
+    if (lone >= 0 && value_key(lr[lone]) == mk) idx = lone;
+    if (grp >= 0) look(grp, mk);
+    else for (int64_t c0 = tid; c0 < nch; c0 += AU * NT) look(c0, mk);
+  }
+  for (int o = 32; o >= 1; o >>= 1) idx = min(idx, (int64_t)__shfl_xor(idx, o, 64));
+  if (lane == 0) si[wave] = idx;
+  __syncthreads();
+  if (tid == 0) {
+    for (int i = 1; i < NT / 64; ++i) idx = min(idx, si[i]);
+    st_agent(out + blockIdx.x, idx);
   }
   stores_done();
 }

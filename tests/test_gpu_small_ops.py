@@ -187,6 +187,27 @@ def test_argmax(ops, dev):
     assert out[2] == 1234
 
 
+@pytest.mark.parametrize("vocab", [1, 7, 8, 17, 8191, 65543])
+@pytest.mark.parametrize("kind", ["randn", "zeros", "ties", "nan", "-inf"])
+def test_argmax_edges(ops, dev, vocab, kind):
+    """Rows that start 2 to 14 bytes past a 16-byte boundary, single elements
+    around the chunks, zeros of both signs (equal), NaN of both signs (first
+    one wins), the lowest value everywhere."""
+    rng = np.random.default_rng(vocab)
+    x = randn_bf16(rng, (8, vocab))
+    if kind == "zeros":
+        x &= 0x8000
+    elif kind == "ties":
+        x = f32_to_bf16_bits(rng.integers(-3, 3, (8, vocab)).astype(np.float32))
+    elif kind == "nan":
+        x[:, vocab // 2], x[:, vocab - 1] = 0xFFC0, 0x7FC0
+    elif kind == "-inf":
+        x[:] = 0xFF80
+    f = bf16_bits_to_f32(x)
+    want = [int(np.argmax(np.isnan(r))) if np.isnan(r).any() else int(np.argmax(r)) for r in f]
+    assert ops.argmax(bf16_dev(x, dev)).cpu().tolist() == want
+
+
 def test_argmax_ragged_vocab(ops, dev):
     """vocab 1003: row 0 is 16-byte aligned (chunks of 8 values, then a
     3-element tail), the other rows are not (element by element)."""
