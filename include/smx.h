@@ -39,7 +39,7 @@
 extern "C" {
 #endif
 
-#define SMX_ABI_VERSION 10
+#define SMX_ABI_VERSION 11
 
 /* Return codes besides 0 and hipError_t values. */
 #define SMX_EINVAL 10001      /* an argument failed validation */
@@ -413,6 +413,21 @@ int smx_compute_slot_mapping(void* stream, const int32_t* query_start_loc, int32
  */
 int smx_q4_0_gemm(void* stream, const void* x, const void* w, void* y, int64_t m, int64_t n,
                   int64_t k);
+
+/*
+ * Q4_0 GEMM for any number of activation rows and any k % 32 == 0: y[m, n] =
+ * x[m, k] W^T, fp32 accumulation, bf16 out.  Up to 16 rows multiply the exact
+ * weights (smx_q4_0_gemv's arithmetic), more take their bf16 roundings (the
+ * values of smx_q4_0_dequant_bf16).  x 16-byte aligned, w 4-byte aligned,
+ * m * k < 2^30.
+ */
+int smx_q4_0_gemm_rows(void* stream, const void* x, const void* w, void* y, int64_t m, int64_t n,
+                       int64_t k);
+
+/* Whether smx_q4_0_gemm_rows is the faster way for these sizes (1), or
+ * smx_q4_0_dequant_bf16 and a library GEMM (0; also for m <= 16 and for sizes
+ * smx_q4_0_gemm_rows does not take). */
+int smx_q4_0_gemm_rows_preferred(int64_t m, int64_t n, int64_t k);
 
 /*
  * smx_q4_0_gemm with the SwiGLU epilogue: w holds 2d rows (gate rows 0..d-1,

@@ -23,10 +23,15 @@ same hook for Q4_0 linears on vLLM's LinearMethodBase contract:
   apply(layer, x, bias=None) -> [..., N] bf16
       one HIP launch: the Q4_0 GEMV for one activation row, the MFMA Q4_0
       GEMM for 2..16 rows (K % 64 == 0; over the packed weights when pack()
-      made them); more rows (prefill) go through the
-      bf16 weights the reference's stock path uses (dequantised on the
-      device, then a library GEMM), as Q6HeadMethod defers to the stock
-      method outside its one-row case.  Bias added after.
+      made them; any other K: q4_0_gemm_rows, small matrices the GEMV per
+      row).  More rows (prefill) multiply
+      the bf16 weights the reference's stock path uses, as Q6HeadMethod
+      defers to the stock method outside its one-row case: up to a few
+      hundred rows in one launch that converts the weights as it reads them
+      (q4_0_gemm_rows, where torch_ops.gemm_rows_preferred says it is the
+      faster way), else, and where torch has to see the product (autograd,
+      functorch transforms, autocast), dequantised on the device, then a
+      library GEMM.  Bias added after.
 
 vLLM is not installed in this image; when it is, the class derives from its
 LinearMethodBase so vLLM's loaders accept it unchanged.
@@ -54,6 +59,12 @@ except Exception:  # noqa: BLE001
 
 #: activation rows one MFMA Q4_0 GEMM launch serves (the kernel's m limit)
 GEMM_MAX_ROWS = 16
+
+#: weights (n * k) from which q4_0_gemm_rows takes a call.  Smaller matrices
+#: keep the launches that callers and the boundary tests know for them (the GEMV
+#: per row, dequantisation and the library), where the device's time hides behind
+#: the host's (1024 x 2560 at 40 rows: 14.6 us, fused 6.4)
+GEMM_ROWS_MIN_WEIGHTS = 3_000_000
 
 
 class Q4_0Config:
@@ -140,14 +151,19 @@ class Q4_0LinearMethod(_Base):
         elif m == 1:
             out = torch_ops.q4_0_gemv(rows, w, n, k)
         elif m <= GEMM_MAX_ROWS and k % 64 == 0:
-            if rows.data_ptr() % 16:
-                rows = rows.clone()  # the tile kernel stages 16-byte activation chunks
-            out = torch_ops.q4_0_gemm(rows, gemm_weight(layer), n, k)
+            out = torch_ops.q4_0_gemm(_aligned16(rows), gemm_weight(layer), n, k)
+        elif m <= GEMM_MAX_ROWS and n * k >= GEMM_ROWS_MIN_WEIGHTS and w.data_ptr() % 4 == 0:
+            # K % 64 != 0: one launch for all rows (4001 x 2592, 5 rows: 5.5 us;
+            # the GEMV below is 5.8 us for each)
+            out = torch_ops.q4_0_gemm_rows(_aligned16(rows), w, n, k)
         elif m <= GEMM_MAX_ROWS:
-            # K % 64 != 0: the GEMV (any K % 32 == 0), one launch per row
+            # the GEMV (any K % 32 == 0, 2-byte aligned), one launch per row
             out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
             for i in range(m):
                 torch_ops.q4_0_gemv(rows[i], w, n, k, out=out[i])
+        elif (n * k >= GEMM_ROWS_MIN_WEIGHTS and w.data_ptr() % 4 == 0
+              and torch_ops.gemm_rows_preferred(m, n, k) and not _torch_sees(rows)):
+            out = torch_ops.q4_0_gemm_rows(_aligned16(rows), w, n, k)
         else:
             w_bf16 = torch_ops.q4_0_dequant_bf16(w, n, k)
             out = torch.nn.functional.linear(rows, w_bf16.view(n, k))
@@ -165,6 +181,24 @@ class Q4_0LinearMethod(_Base):
             raise ValueError("apply_swiglu needs a merged [gate, up] layer of equal halves")
         return torch_ops.q4_0_gemv_swiglu(x.reshape(-1), layer.qweight.reshape(-1), sizes[0],
                                           layer.q4_0_k, out=out)
+
+
+def _aligned16(rows: torch.Tensor) -> torch.Tensor:
+    """The GEMM kernels stage activations in 16-byte chunks."""
+    return rows.clone() if rows.data_ptr() % 16 else rows
+
+
+def _torch_sees(rows: torch.Tensor) -> bool:
+    """Whether a product of `rows` has to be a torch operation: autograd or a
+    forward-mode level records it, a functorch transform or a tensor subclass
+    or mode intercepts it, or autocast chooses its type."""
+    return (rows.requires_grad and torch.is_grad_enabled()
+            or torch.is_autocast_enabled("cuda")
+            or type(rows) not in (torch.Tensor, torch.nn.Parameter)
+            or torch.autograd.forward_ad._current_level >= 0
+            or torch._C._functorch.maybe_current_level() is not None
+            or torch._C._len_torch_dispatch_stack() > 0
+            or torch._C._len_torch_function_stack() > 0)
 
 
 def gemm_weight(layer: torch.nn.Module, gated: bool = False):

@@ -29,7 +29,7 @@ DEFAULT_RECORD = LIB_PATH.with_name("libsmx.validation.json")
 #: benchmark and the build check do (they are what validates and measures the
 #: library as built); a record named by SMX_VALIDATION_RECORD is still checked
 UNVALIDATED_ENV = "SMX_ALLOW_UNVALIDATED"
-ABI_VERSION = 10
+ABI_VERSION = 11
 SMX_EINVAL = 10001
 SMX_EUNSUPPORTED = 10002
 
@@ -63,6 +63,8 @@ SIGNATURES = {
                                                       _P, _I32, _I32, _I32, _I32, _I32, _I32,
                                                       _I32, _I32, _I32, _I32, _F32, _F32],
     "smx_q4_0_gemm": [_P, _P, _P, _P, _I64, _I64, _I64],
+    "smx_q4_0_gemm_rows": [_P, _P, _P, _P, _I64, _I64, _I64],
+    "smx_q4_0_gemm_rows_preferred": [_I64, _I64, _I64],
     "smx_q4_0_gemm_swiglu": [_P, _P, _P, _P, _I64, _I64, _I64],
     "smx_q4_0_gemm_gelu": [_P, _P, _P, _P, _P, _I64, _I64, _I64],
     "smx_q4_0_gemm_argmax": [_P, _P, _P, _P, _P, _I64, _I64, _I64],

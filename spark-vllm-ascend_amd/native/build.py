@@ -39,8 +39,8 @@ COMMON = [
     # preloading): no scalar-load round trip before a kernel's first loads
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
 ]
-SOURCES = ["q4_0_gemv.hip", "q4_0_gemm.hip", "splitkv_attention.hip", "small_ops.hip",
-           "abi.cpp", "step_runner.cpp"]
+SOURCES = ["q4_0_gemv.hip", "q4_0_gemm.hip", "q4_0_gemm_rows.hip", "splitkv_attention.hip",
+           "small_ops.hip", "abi.cpp", "step_runner.cpp"]
 DEVICE_SOURCES = [s for s in SOURCES if s.endswith(".hip")]
 
 

@@ -668,6 +668,29 @@ def q4_0_gemm(x: torch.Tensor, w: torch.Tensor | PackedQ4_0, n: int, k: int,
     return out
 
 
+def q4_0_gemm_rows(x: torch.Tensor, w: torch.Tensor, n: int, k: int,
+                   out: torch.Tensor | None = None) -> torch.Tensor:
+    """y [m, n] = x [m, k] . W^T for any m >= 1 and any k % 32 == 0, W GGUF Q4_0
+    (m <= 16: the exact weights; more rows: their bf16 roundings)."""
+    _need(k % 32 == 0 and k > 0 and n > 0, "need n > 0 and k a positive multiple of 32")
+    _need(x.dim() == 2 and x.shape[0] >= 1 and x.shape[1] == k, "x must be [m, k]")
+    _check(x, "x", BF16)
+    _need(x.data_ptr() % 16 == 0, "x must be 16-byte aligned")
+    _check(w, "w", torch.uint8, n * q4_0_row_bytes(k), x.device)
+    if out is None:
+        out = torch.empty((x.shape[0], n), dtype=BF16, device=x.device)
+    _check(out, "out", BF16, x.shape[0] * n, x.device)
+    call("smx_q4_0_gemm_rows", _stream(x), x.data_ptr(), w.data_ptr(), out.data_ptr(),
+         x.shape[0], n, k)
+    return out
+
+
+def gemm_rows_preferred(m: int, n: int, k: int) -> bool:
+    """Whether q4_0_gemm_rows beats dequantisation + a library GEMM (m > 16)."""
+    from . import load
+    return bool(load().smx_q4_0_gemm_rows_preferred(m, n, k))
+
+
 def q4_0_gemm_swiglu(x: torch.Tensor, w: torch.Tensor | PackedQ4_0, d: int, k: int,
                      out: torch.Tensor | None = None,
                      lut: torch.Tensor | None = None) -> torch.Tensor:

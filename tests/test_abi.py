@@ -90,6 +90,11 @@ def test_bindings_cover_header():
     ("smx_q4_0_gemm", (None, 16, 16, 16, 4, 64, 96)),
     ("smx_q4_0_gemm_swiglu", (None, 12, 16, 16, 4, 64, 256)),
     ("smx_compute_slot_mapping", (None, 16, 0, 16, 16, 16, 1, 4, 8, 128)),
+    ("smx_q4_0_gemm_rows", (None, 16, 16, 16, 0, 64, 256)),
+    ("smx_q4_0_gemm_rows", (None, 16, 16, 16, 20, 64, 48)),
+    ("smx_q4_0_gemm_rows", (None, 24, 16, 16, 20, 64, 256)),
+    ("smx_q4_0_gemm_rows", (None, 16, 18, 16, 20, 64, 256)),
+    ("smx_q4_0_gemm_rows", (None, 16, 16, 16, 1 << 19, 64, 1 << 11)),
     ("smx_qknorm_rope_splitkv_decode_merged",
      (None, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 16, 1, 4, 8, 8, 128, 32, 8, 128, 0, 1e-6, 0.1)),
     ("smx_qknorm_rope_splitkv_decode_merged",

@@ -1,0 +1,144 @@
+"""GPU parity of smx_q4_0_gemm_rows (any row count, any K % 32 == 0): against
+float64 products of the weights it multiplies (exact up to 16 rows, their bf16
+roundings above), one-hot activations that must select weights bit for bit
+(which pins the lane transposes, the two alignments of a block and the last
+block of the matrix), every launch shape, and the linear that routes to it."""
+import numpy as np
+import pytest
+
+from oracle import q4_0 as oq
+from oracle.bf16 import bf16_bits_to_f32, f32_to_bf16_bits
+
+from _util import bf16_dev, bits_of, f32_of, pkg, randn_bf16
+
+pytestmark = pytest.mark.gpu
+
+# (n, k) odd in each way: fewer columns than a tile, an odd number of blocks in
+# the matrix (its last block read 2 bytes early), K of 1..3 blocks past a tile
+SIZES = [(1, 32), (33, 96), (50, 160), (97, 32), (131, 2592), (256, 2560)]
+
+
+@pytest.fixture(scope="module")
+def dev():
+    import torch
+    return torch.device("cuda:0")
+
+
+@pytest.fixture(scope="module")
+def ops():
+    return pkg("native.torch_ops")
+
+
+def _w(blocks, dev):
+    import torch
+    return torch.from_numpy(np.ascontiguousarray(blocks).reshape(-1)).to(dev)
+
+
+def _weights(blocks, n, k, rows):
+    w = oq.dequant_f32(blocks, n, k).reshape(n, k)
+    return w if rows <= 16 else bf16_bits_to_f32(f32_to_bf16_bits(w))
+
+
+def _check(y, x, w):
+    """fp32 sums of k products in any order (k 2^-24 of the absolute sum),
+    rounded to bf16 (2^-8 covers the half ulp of 2^-9 either way)."""
+    x64, w64 = bf16_bits_to_f32(x).astype(np.float64), w.astype(np.float64)
+    ref = x64 @ w64.T
+    bound = 2.0 ** -8 * np.abs(ref) + x.shape[1] * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
+    bad = np.abs(y - ref) > bound
+    assert not bad.any(), (np.argwhere(bad)[:4], y[bad][:4], ref[bad][:4])
+
+
+@pytest.mark.parametrize("n,k", SIZES)
+@pytest.mark.parametrize("m", [1, 5, 16, 17, 48, 65, 193, 257])
+def test_rows_vs_float64(ops, dev, m, n, k):
+    blocks = oq.make_blocks(n, k, seed=n + k + m)
+    x = randn_bf16(np.random.default_rng(m + n + k), (m, k))
+    y = f32_of(ops.q4_0_gemm_rows(bf16_dev(x, dev), _w(blocks, dev), n, k)).reshape(m, n)
+    _check(y, x, _weights(blocks, n, k, m))
+
+
+@pytest.mark.parametrize("n,k", SIZES)
+@pytest.mark.parametrize("m", [16, 40])
+def test_rows_one_hot_bits_and_bounds(ops, dev, m, n, k):
+    import torch
+    blocks = oq.make_blocks(n, k, seed=n, scale=1.0)
+    cols = (np.arange(m) * 37 + k - m) % k
+    x = np.zeros((m, k), dtype=np.uint16)
+    x[np.arange(m), cols] = f32_to_bf16_bits(np.float32([1.0]))[0]
+    y = torch.full((m * n + 64,), 7.0, dtype=torch.bfloat16, device=dev)
+    ops.q4_0_gemm_rows(bf16_dev(x, dev), _w(blocks, dev), n, k, out=y[:m * n])
+    want = f32_to_bf16_bits(oq.dequant_f32(blocks, n, k).reshape(n, k)[:, cols].T + np.float32(0))
+    np.testing.assert_array_equal(bits_of(y)[:m * n].reshape(m, n) & 0x7FFF, want & 0x7FFF)
+    np.testing.assert_array_equal(f32_of(y)[:m * n].reshape(m, n), bf16_bits_to_f32(want))
+    assert (y[m * n:] == 7.0).all()
+
+
+def test_rows_every_launch_shape():
+    """Each launch shape, forced through its tuning switch (read once per
+    process, so one child process runs them all)."""
+    import subprocess
+    import sys
+    from pathlib import Path
+    code = """
+import os
+os.environ.update(SMX_TUNE="1", SMX_ALLOW_UNVALIDATED="1")
+import importlib
+import torch
+import __graft_entry__
+ops = importlib.import_module(__graft_entry__.load_package().__name__ + ".native.torch_ops")
+g = torch.Generator(device="cuda")
+g.manual_seed(1)
+for m, n, k in ((17, 130, 416), (150, 77, 1056)):
+    w = torch.randint(0, 60, (n * k // 32 * 18,), generator=g, device="cuda", dtype=torch.uint8)
+    x = torch.randn((m, k), generator=g, device="cuda").to(torch.bfloat16)
+    wd, xd = ops.q4_0_dequant_bf16(w, n, k).cpu().double(), x.cpu().double()
+    ref = xd @ wd.T
+    bound = 2.0 ** -8 * ref.abs() + k * 2.0 ** -24 * (xd.abs() @ wd.abs().T)
+    for shape in range(14):
+        os.environ["SMX_ROWS_SHAPE"] = str(shape)
+        print(m, n, k, shape, flush=True)
+        y = ops.q4_0_gemm_rows(x, w, n, k).cpu().double()
+        assert ((y - ref).abs() <= bound).all(), (m, n, k, shape)
+print("ok")
+"""
+    r = subprocess.run([sys.executable, "-c", code], capture_output=True, text=True, timeout=100,
+                       cwd=Path(__file__).resolve().parent.parent)
+    assert r.returncode == 0 and r.stdout.strip().endswith("ok"), r.stdout[-200:] + r.stderr[-800:]
+
+
+def test_rows_infinities(ops, dev):
+    """An infinite activation gives what a product with the weights gives."""
+    n, k, m = 48, 256, 20
+    blocks = oq.make_blocks(n, k, seed=3)
+    x = randn_bf16(np.random.default_rng(4), (m, k))
+    x[3, 100], x[7, 5] = 0x7F80, 0xFF80
+    with np.errstate(invalid="ignore"):
+        ref = bf16_bits_to_f32(x).astype(np.float64) @ _weights(blocks, n, k, m).astype(np.float64).T
+    for rows in (m, 8):
+        y = f32_of(ops.q4_0_gemm_rows(bf16_dev(x[:rows], dev), _w(blocks, dev), n, k))
+        y = y.reshape(rows, n)
+        np.testing.assert_array_equal(np.isnan(y), np.isnan(ref[:rows]))
+        np.testing.assert_array_equal(np.isposinf(y), np.isposinf(ref[:rows]))
+
+
+def test_linear_routes(dev):
+    """Rows that torch only multiplies take the fused kernel, rows that
+    autograd records keep the library product and its gradient."""
+    import torch
+    lin = pkg("integration.linear")
+    n, k, m = 4001, 2592, 40
+    layer = lin.Q4_0Linear(k, [n], device=dev)
+    blocks = oq.make_blocks(n, k, seed=5)
+    layer.qweight.data.copy_(_w(blocks, dev).view(n, -1))
+    x = bf16_dev(randn_bf16(np.random.default_rng(6), (m, k)), dev).view(m, k)
+    y = layer(x)
+    xg = x.clone().requires_grad_(True)
+    yg = layer(xg)
+    assert yg.requires_grad
+    yg.float().sum().backward()
+    assert xg.grad is not None and not y.requires_grad
+    torch.testing.assert_close(y.float(), yg.detach().float(), rtol=2.0 ** -6, atol=1e-2)
+    off = torch.empty(m * k + 1, dtype=torch.bfloat16, device=dev)[1:].view(m, k).copy_(x)
+    assert torch.equal(layer(off), y)  # 2-byte aligned rows
+    assert torch.equal(layer(off[:5]), layer(x[:5]))
