@@ -145,7 +145,9 @@ class Q4_0LinearMethod(_Base):
             raise ValueError(f"expected bf16 activations, got {x.dtype}")
         rows = x.reshape(-1, k).contiguous()
         m = rows.shape[0]
-        w = layer.qweight.reshape(-1)
+        w = layer.qweight
+        if not w.is_contiguous():
+            w = w.contiguous()
         if m == 0:
             out = torch.empty((0, n), dtype=torch.bfloat16, device=x.device)
         elif m == 1:
@@ -167,7 +169,8 @@ class Q4_0LinearMethod(_Base):
         else:
             w_bf16 = torch_ops.q4_0_dequant_bf16(w, n, k)
             out = torch.nn.functional.linear(rows, w_bf16.view(n, k))
-        out = out.reshape(*x.shape[:-1], n)
+        if x.dim() != 2:
+            out = out.reshape(*x.shape[:-1], n)
         if bias is not None:
             out = out + bias
         return out

@@ -12,13 +12,15 @@ from __future__ import annotations
 
 import torch
 
-from . import call
+from . import call, load
 
 BF16 = torch.bfloat16
 
 
 def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
+    """The current HIP stream of the tensor's device.  (The raw getter: 0.14 us;
+    torch.cuda.current_stream() builds a Stream object for its handle, 2.0 us.)"""
+    return torch._C._cuda_getCurrentRawStream(t.get_device())
 
 
 def _need(cond: bool, msg: str) -> None:
@@ -28,6 +30,14 @@ def _need(cond: bool, msg: str) -> None:
 
 def _check(t: torch.Tensor, name: str, dtype: torch.dtype, numel: int | None = None,
            device: torch.device | None = None) -> None:
+    # one condition for a valid tensor; what is wrong is worked out, and its
+    # message formatted, only for one that is not (a call makes up to 13 checks)
+    if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype == dtype and t.is_contiguous()
+            and (numel is None or t.numel() == numel) and (device is None or t.device == device)):
+        _refuse(t, name, dtype, numel, device)
+
+
+def _refuse(t, name, dtype, numel, device) -> None:
     _need(isinstance(t, torch.Tensor), f"{name} must be a tensor")
     _need(t.is_cuda, f"{name} must be on a GPU device")
     _need(t.dtype == dtype, f"{name} must be {dtype}, got {t.dtype}")
@@ -36,6 +46,7 @@ def _check(t: torch.Tensor, name: str, dtype: torch.dtype, numel: int | None = N
         _need(t.numel() == numel, f"{name} must have {numel} elements, got {t.numel()}")
     if device is not None:
         _need(t.device == device, f"{name} must be on {device}, got {t.device}")
+    raise ValueError(f"{name} is not a valid argument")
 
 
 def q4_0_row_bytes(k: int) -> int:
@@ -120,7 +131,7 @@ def splitkv_decode(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor
     num_seqs, n_q, hd = q.shape
     num_blocks, bs, n_kv, hd2 = k_cache.shape
     _need(hd == hd2, "head_dim mismatch between q and the cache")
-    _need(tuple(v_cache.shape) == tuple(k_cache.shape), "k_cache and v_cache shapes differ")
+    _need(v_cache.shape == k_cache.shape, "k_cache and v_cache shapes differ")
     _check(q, "q", BF16)
     _check(k_cache, "k_cache", BF16, device=q.device)
     _check(v_cache, "v_cache", BF16, device=q.device)
@@ -149,7 +160,7 @@ def splitkv_decode_merged(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch
     num_seqs, n_q, hd = q.shape
     num_blocks, bs, n_kv, hd2 = k_cache.shape
     _need(hd == hd2, "head_dim mismatch between q and the cache")
-    _need(tuple(v_cache.shape) == tuple(k_cache.shape), "k_cache and v_cache shapes differ")
+    _need(v_cache.shape == k_cache.shape, "k_cache and v_cache shapes differ")
     _check(q, "q", BF16)
     _check(k_cache, "k_cache", BF16, device=q.device)
     _check(v_cache, "v_cache", BF16, device=q.device)
@@ -227,7 +238,7 @@ def splitkv_decode_planned_merged(q: torch.Tensor, k_cache: torch.Tensor, v_cach
     num_seqs, n_q, hd = q.shape
     num_blocks, bs, n_kv, hd2 = k_cache.shape
     _need(hd == hd2, "head_dim mismatch between q and the cache")
-    _need(tuple(v_cache.shape) == tuple(k_cache.shape), "k_cache and v_cache shapes differ")
+    _need(v_cache.shape == k_cache.shape, "k_cache and v_cache shapes differ")
     _check(q, "q", BF16)
     _check(k_cache, "k_cache", BF16, device=q.device)
     _check(v_cache, "v_cache", BF16, device=q.device)
@@ -287,7 +298,7 @@ def qknorm_rope_kv_write(qkv: torch.Tensor, q_gamma: torch.Tensor, k_gamma: torc
     _check(slot_mapping, "slot_mapping", torch.int64, num_tokens, qkv.device)
     _check(k_cache, "k_cache", BF16, device=qkv.device)
     _check(v_cache, "v_cache", BF16, device=qkv.device)
-    _need(tuple(v_cache.shape) == tuple(k_cache.shape), "k_cache and v_cache shapes differ")
+    _need(v_cache.shape == k_cache.shape, "k_cache and v_cache shapes differ")
     if q_out is None:
         q_out = torch.empty((num_tokens, n_q, hd), dtype=BF16, device=qkv.device)
     _check(q_out, "q_out", BF16, num_tokens * n_q * hd, qkv.device)
@@ -357,7 +368,7 @@ def reshape_and_cache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Ten
     _check(value, "value", BF16, num_tokens * n_kv * hd, key.device)
     _check(k_cache, "k_cache", BF16, device=key.device)
     _check(v_cache, "v_cache", BF16, device=key.device)
-    _need(tuple(v_cache.shape) == tuple(k_cache.shape), "k_cache and v_cache shapes differ")
+    _need(v_cache.shape == k_cache.shape, "k_cache and v_cache shapes differ")
     _check(slot_mapping, "slot_mapping", torch.int64, num_tokens, key.device)
     call("smx_reshape_and_cache", _stream(key), key.data_ptr(), value.data_ptr(),
          k_cache.data_ptr(), v_cache.data_ptr(), slot_mapping.data_ptr(), num_tokens, n_kv, hd,
@@ -478,7 +489,6 @@ def add_rmsnorm_gemv_gelu(x: torch.Tensor, residual: torch.Tensor | None, gamma:
 
 
 def argmax_keys_size(n: int, k: int) -> int:
-    from . import load
     return int(load().smx_q4_0_argmax_keys_size(n, k))
 
 
@@ -520,7 +530,7 @@ def qknorm_rope_splitkv_decode_merged(qkv: torch.Tensor, q_gamma: torch.Tensor,
     _check(slot_mapping, "slot_mapping", torch.int64, num_seqs, qkv.device)
     _check(k_cache, "k_cache", BF16, device=qkv.device)
     _check(v_cache, "v_cache", BF16, device=qkv.device)
-    _need(tuple(v_cache.shape) == tuple(k_cache.shape), "k_cache and v_cache shapes differ")
+    _need(v_cache.shape == k_cache.shape, "k_cache and v_cache shapes differ")
     _check(block_table, "block_table", torch.int32, device=qkv.device)
     _need(block_table.dim() == 2 and block_table.shape[0] == num_seqs, "block_table must be [seqs, max_blocks]")
     _check(seq_lens, "seq_lens", torch.int32, num_seqs, qkv.device)
@@ -556,7 +566,7 @@ def qknorm_rope_splitkv_decode_planned_merged(qkv: torch.Tensor, q_gamma: torch.
     _need(cos_sin.dim() == 2 and cos_sin.shape[1] == hd, "cos_sin must be [max_position, head_dim]")
     _check(k_cache, "k_cache", BF16, device=qkv.device)
     _check(v_cache, "v_cache", BF16, device=qkv.device)
-    _need(tuple(v_cache.shape) == tuple(k_cache.shape), "k_cache and v_cache shapes differ")
+    _need(v_cache.shape == k_cache.shape, "k_cache and v_cache shapes differ")
     _check(block_table, "block_table", torch.int32, device=qkv.device)
     _need(block_table.dim() == 2, "block_table must be [seqs, max_blocks]")
     _check(plan, "plan", torch.int32, (num_items + num_seqs) * PLAN_WORDS, qkv.device)
@@ -616,7 +626,6 @@ class PackedQ4_0:
 def q4_0_packed_bytes(n: int, k: int, gated: bool = False) -> int:
     """Bytes of the packed form of an [n, k] Q4_0 matrix (gated: [2n, k]);
     -1 when unsupported (k not a positive multiple of 256)."""
-    from . import load
     return int(load().smx_q4_0_packed_bytes(n, k, 1 if gated else 0))
 
 
@@ -638,13 +647,14 @@ def q4_0_repack(w: torch.Tensor, n: int, k: int, gated: bool = False,
 def _gemm_x(x: torch.Tensor, k: int, align: int) -> None:
     _need(x.dim() == 2 and x.shape[1] == k and 1 <= x.shape[0] <= 16, "x must be [m <= 16, k]")
     _check(x, "x", BF16)
-    _need(x.data_ptr() % align == 0, f"x must be {align}-byte aligned")
+    if x.data_ptr() % align:
+        raise ValueError(f"x must be {align}-byte aligned")
 
 
 def _packed_checked(w: PackedQ4_0, n: int, k: int, gated: bool, device) -> int:
-    _need(w.n == n and w.k == k and w.gated == gated,
-          f"packed weights hold [{w.n}, {w.k}] (gated={w.gated}), the call wants [{n}, {k}] "
-          f"(gated={gated})")
+    if not (w.n == n and w.k == k and w.gated == gated):
+        raise ValueError(f"packed weights hold [{w.n}, {w.k}] (gated={w.gated}), the call wants "
+                         f"[{n}, {k}] (gated={gated})")
     _check(w.data, "w.data", torch.uint8, q4_0_packed_bytes(n, k, gated), device)
     return w.data.data_ptr()
 
@@ -687,7 +697,6 @@ def q4_0_gemm_rows(x: torch.Tensor, w: torch.Tensor, n: int, k: int,
 
 def gemm_rows_preferred(m: int, n: int, k: int) -> bool:
     """Whether q4_0_gemm_rows beats dequantisation + a library GEMM (m > 16)."""
-    from . import load
     return bool(load().smx_q4_0_gemm_rows_preferred(m, n, k))
 
 
@@ -728,7 +737,6 @@ def q4_0_gemm_gelu(x: torch.Tensor, w: torch.Tensor | PackedQ4_0, lut: torch.Ten
 
 def gemm_keys_per_row(n: int) -> int:
     """Greedy-argmax keys q4_0_gemm_argmax writes per row (one per 16 outputs)."""
-    from . import load
     return int(load().smx_q4_0_gemm_keys_per_row(n))
 
 
