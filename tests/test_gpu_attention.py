@@ -337,3 +337,59 @@ def test_backend_forward(dev, planned):
         ref = oatt.attention_f64(qf[i], oatt.gather_paged(kf, table[i], L),
                                  oatt.gather_paged(vf, table[i], L), HD ** -0.5)
         assert_attention_close(got[i], ref, f"sequence {i}")
+
+
+@pytest.mark.parametrize("fused", [False, True])
+def test_plan_one_wave_per_workgroup(ops, dev, fused):
+    """At least 512 live workgroups and splits of 768 tokens: one wave walks a
+    split (70 items here; 40 are just below, four waves): against capacity
+    splits of the same inputs, the new token's K/V included."""
+    import torch
+    att = pkg("integration.attention")
+    n_kv, n_q, hd, bs, splits = 8, 32, 128, 128, 32
+    lens = [13000, 12801, 12289, 12161]
+    S, per_seq = len(lens), 104
+    g = torch.Generator(device=dev)
+    g.manual_seed(3)
+    table = torch.randperm(S * per_seq, generator=g, device=dev).to(torch.int32).view(S, per_seq)
+    kv = torch.randn((2, S * per_seq, bs, n_kv, hd), generator=g, device=dev).to(torch.bfloat16)
+    L = torch.tensor(lens, dtype=torch.int32, device=dev)
+    pos = (L - 1).long()
+    slots = table[torch.arange(S, device=dev), pos // bs].long() * bs + pos % bs
+    scale = hd ** -0.5
+    outs, caches = [], []
+    for items in (0, 40, 70):  # capacity splits, 4 waves, 1 wave
+        c = kv.clone()
+        po, pl = att.split_partials(S, splits, n_q, hd, dev)
+        plan = None
+        if items:
+            plan = ops.splitkv_plan(L, table, bs, items, po, pl, positions=pos,
+                                    slot_mapping=slots)
+            assert int((plan[:, 0] >= 0).sum()) * n_kv >= 512 if items == 70 else True
+        if fused:
+            gq = torch.Generator(device=dev)
+            gq.manual_seed(4)
+            qkv = torch.randn((S, (n_q + 2 * n_kv) * hd), generator=gq, device=dev).to(torch.bfloat16)
+            gamma = torch.ones(hd, dtype=torch.bfloat16, device=dev)
+            cos_sin = torch.rand((per_seq * bs, hd), generator=gq, device=dev).to(torch.bfloat16)
+            if items:
+                out = ops.qknorm_rope_splitkv_decode_planned_merged(
+                    qkv, gamma, gamma, cos_sin, c[0], c[1], table, plan, items, scale, 1e-6, n_q,
+                    po, pl)
+            else:
+                out = ops.qknorm_rope_splitkv_decode_merged(
+                    qkv, gamma, gamma, cos_sin, pos, slots, c[0], c[1], table, L, splits, scale,
+                    1e-6, n_q, po, pl)
+        else:
+            g5 = torch.Generator(device=dev)
+            g5.manual_seed(5)
+            q = torch.randn((S, n_q, hd), generator=g5, device=dev).to(torch.bfloat16)
+            out = (ops.splitkv_decode_planned_merged(q, c[0], c[1], table, plan, items, scale, po, pl)
+                   if items else
+                   ops.splitkv_decode_merged(q, c[0], c[1], table, L, splits, scale, po, pl))
+        outs.append(out.float().clone())
+        caches.append(c)
+    for o, c in zip(outs[1:], caches[1:]):
+        # bf16 probabilities at other running maxima: 2^-8 of the output's own size
+        torch.testing.assert_close(o, outs[0], rtol=2.0 ** -6, atol=2.0 ** -6 * float(outs[0].std()))
+        assert torch.equal(c, caches[0])
