@@ -390,6 +390,15 @@ int smx_argmax_bf16(void* stream, const void* logits, int64_t rows,
                     int64_t vocab, int64_t* out_ids);
 
 /*
+ * smx_argmax_bf16 by two launches with a workspace between them: keys
+ * [rows, smx_argmax_parts(vocab)] uint64, num_keys their number.  The faster way
+ * where smx_argmax_parts is not 0 (a row is then too long for one workgroup).
+ */
+int64_t smx_argmax_parts(int64_t vocab);
+int smx_argmax_bf16_parts(void* stream, const void* logits, int64_t rows, int64_t vocab,
+                          uint64_t* keys, int64_t num_keys, int64_t* out_ids);
+
+/*
  * Slot mapping of a ragged batch (vLLM's compute_slot_mapping for one KV
  * group): token t of request r (query_start_loc[r] <= t <
  * query_start_loc[r + 1], int32 [num_reqs + 1]) at positions[t] gets

@@ -83,6 +83,8 @@ SIGNATURES = {
     "smx_gelu_mul": [_P, _P, _P, _P, _I64, _I64],
     "smx_embedding": [_P, _P, _P, _P, _I64, _I64, _I64],
     "smx_argmax_bf16": [_P, _P, _I64, _I64, _P],
+    "smx_argmax_parts": [_I64],
+    "smx_argmax_bf16_parts": [_P, _P, _I64, _I64, _P, _I64, _P],
     "smx_reshape_and_cache": [_P, _P, _P, _P, _P, _P, _I32, _I32, _I32, _I32, _I32],
     "smx_decode_advance": [_P, _P, _P, _I32, _P, _P, _P, _P, _P, _P, _P, _P, _I32, _I32, _I32,
                            _I32, _P, _P, _I64, _I64],
@@ -108,7 +110,8 @@ RUNNER_FENCES_AGENT = 0
 RUNNER_FENCES_ACQUIRE_ONLY = 1
 
 # return types other than int
-RESTYPES = {"smx_q4_0_argmax_keys_size": ctypes.c_int64,
+RESTYPES = {"smx_argmax_parts": ctypes.c_int64,
+            "smx_q4_0_argmax_keys_size": ctypes.c_int64,
             "smx_q4_0_gemm_keys_per_row": ctypes.c_int64,
             "smx_q4_0_packed_bytes": ctypes.c_int64,
             "smx_runner_destroy": None}

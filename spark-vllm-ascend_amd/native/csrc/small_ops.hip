@@ -344,18 +344,29 @@ __device__ __forceinline__ int value_key(uint32_t h16) {
 // thread's maximum first rose to its value; then the threads that hold the row's
 // maximum look for its index in their group alone.  (Comparing (value, 64-bit
 // index) pairs element by element was bound by one CU's VALU: 25.3 us
-// there, now 11.6.)
+// there, now 11.3.)
 // The elements before the first 16-byte boundary and after the last chunk are
 // one per thread.  A NaN anywhere in the row sends it through an
 // element-by-element scan of the keys that order NaN.
-__global__ __launch_bounds__(1024) void argmax_kernel(const uint16_t* __restrict__ logits,
-                                                      int64_t vocab, int64_t* __restrict__ out) {
-  constexpr int NT = 1024;  // threads per workgroup
-  constexpr int AU = 8;     // chunks per thread and group
+//
+// PARTS: workgroup (p, row) takes the part_len elements from p * part_len on and
+// leaves their (key, ~index) in keys[row][p] for argmax_keys_kernel: one CU reads
+// 300 KB in 11.3 us whatever it does with them; ARGMAX_PARTS of them and the
+// second launch take 6.2.
+template <int NT, bool PARTS>  // threads per workgroup
+__global__ __launch_bounds__(NT) void argmax_kernel(const uint16_t* __restrict__ logits,
+                                                    int64_t vocab, int64_t* __restrict__ out,
+                                                    int64_t part_len, int parts) {
+  constexpr int AU = 8;  // chunks per thread and group
   __shared__ int sk[NT / 64], sm[NT / 64];
   __shared__ int64_t si[NT / 64];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const uint16_t* lr = logits + (int64_t)blockIdx.x * vocab;
+  const uint16_t* lr = logits + (int64_t)(PARTS ? blockIdx.y : blockIdx.x) * vocab;
+  const int64_t first = PARTS ? blockIdx.x * part_len : 0;
+  if constexpr (PARTS) {
+    lr += first;
+    vocab = min(part_len, vocab - first);  // >= 1: the host makes no empty part
+  }
   const int64_t head = min(vocab, (int64_t)(((0 - (uintptr_t)lr) & 15) >> 1));
   const int64_t nch = (vocab - head) >> 3;
   const int64_t tail = head + 8 * nch;
@@ -430,8 +441,30 @@ __global__ __launch_bounds__(1024) void argmax_kernel(const uint16_t* __restrict
   __syncthreads();
   if (tid == 0) {
     for (int i = 1; i < NT / 64; ++i) idx = min(idx, si[i]);
-    st_agent(out + blockIdx.x, idx);
+    if constexpr (PARTS) {
+      const int k = m > 0x7f80 ? 0x7fff : mk;
+      st_agent(out + (int64_t)blockIdx.y * parts + blockIdx.x,
+               (int64_t)(((uint64_t)(uint32_t)(k + 0x8000) << 32) |
+                         (0xffffffffu - (uint32_t)(first + idx))));
+    } else {
+      st_agent(out + blockIdx.x, idx);
+    }
   }
+  stores_done();
+}
+
+constexpr int ARGMAX_PARTS = 32;  // at most 64: one lane of a wave each
+
+// One wave per row: the largest of its `parts` keys (argmax_kernel).
+__global__ __launch_bounds__(64) void argmax_keys_kernel(const uint64_t* __restrict__ keys,
+                                                         int parts, int64_t* __restrict__ out) {
+  const int lane = threadIdx.x;
+  uint64_t k = keys[(int64_t)blockIdx.x * parts + min(lane, parts - 1)];
+  for (int o = 32; o >= 1; o >>= 1) {
+    const uint64_t other = (uint64_t)__shfl_xor((int64_t)k, o, 64);
+    k = other > k ? other : k;
+  }
+  if (lane == 0) st_agent(out + blockIdx.x, (int64_t)(0xffffffffu - (uint32_t)k));
   stores_done();
 }
 
@@ -725,8 +758,34 @@ extern "C" int smx_argmax_bf16(void* stream, const void* logits, int64_t rows, i
   SMX_REQUIRE(logits && out_ids, "null pointer argument");
   SMX_REQUIRE(rows >= 1 && rows < (1ll << 31) && vocab >= 1, "bad shape");
   SMX_REQUIRE((uintptr_t)out_ids % 8 == 0, "out_ids must be 8-byte aligned");
-  SMX_LAUNCH(smx::argmax_kernel, dim3((unsigned)rows), dim3(1024), 0,
-                     (hipStream_t)stream, (const uint16_t*)logits, vocab, out_ids);
+  SMX_LAUNCH((smx::argmax_kernel<1024, false>), dim3((unsigned)rows), dim3(1024), 0,
+             (hipStream_t)stream, (const uint16_t*)logits, vocab, out_ids, (int64_t)0, 1);
+  return (int)hipGetLastError();
+}
+
+extern "C" int64_t smx_argmax_parts(int64_t vocab) {
+  // From 64K elements on; one workgroup takes 7.0 us for 50000, the two launches 6.
+  if (vocab < 65536 || vocab > 0xffffffffll) return 0;
+  const int64_t len = ((vocab + smx::ARGMAX_PARTS - 1) / smx::ARGMAX_PARTS + 7) / 8 * 8;
+  return (vocab + len - 1) / len;
+}
+
+extern "C" int smx_argmax_bf16_parts(void* stream, const void* logits, int64_t rows,
+                                     int64_t vocab, uint64_t* keys, int64_t num_keys,
+                                     int64_t* out_ids) {
+  SMX_REQUIRE(logits && keys && out_ids, "null pointer argument");
+  SMX_REQUIRE(rows >= 1 && rows <= 65535, "rows must be in [1, 65535]");
+  const int64_t parts = smx_argmax_parts(vocab);
+  SMX_REQUIRE(parts > 0 && num_keys == rows * parts,
+              "num_keys must be rows * smx_argmax_parts(vocab), which is not 0");
+  SMX_REQUIRE((uintptr_t)out_ids % 8 == 0 && (uintptr_t)keys % 8 == 0,
+              "out_ids and keys must be 8-byte aligned");
+  const int64_t len = ((vocab + smx::ARGMAX_PARTS - 1) / smx::ARGMAX_PARTS + 7) / 8 * 8;
+  SMX_LAUNCH((smx::argmax_kernel<256, true>), dim3((unsigned)parts, (unsigned)rows), dim3(256),
+             0, (hipStream_t)stream, (const uint16_t*)logits, vocab, (int64_t*)keys, len,
+             (int)parts);
+  SMX_LAUNCH(smx::argmax_keys_kernel, dim3((unsigned)rows), dim3(64), 0, (hipStream_t)stream,
+             keys, (int)parts, out_ids);
   return (int)hipGetLastError();
 }
 

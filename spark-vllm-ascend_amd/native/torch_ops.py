@@ -355,6 +355,12 @@ def argmax(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tenso
     if out is None:
         out = torch.empty((rows,), dtype=torch.int64, device=logits.device)
     _check(out, "out", torch.int64, rows, logits.device)
+    parts = load().smx_argmax_parts(vocab) if 1 <= rows <= 65535 else 0
+    if parts:
+        keys = torch.empty((rows, parts), dtype=torch.int64, device=logits.device)
+        call("smx_argmax_bf16_parts", _stream(logits), logits.data_ptr(), rows, vocab,
+             keys.data_ptr(), rows * parts, out.data_ptr())
+        return out
     call("smx_argmax_bf16", _stream(logits), logits.data_ptr(), rows, vocab, out.data_ptr())
     return out
 

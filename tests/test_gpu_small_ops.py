@@ -187,7 +187,7 @@ def test_argmax(ops, dev):
     assert out[2] == 1234
 
 
-@pytest.mark.parametrize("vocab", [1, 7, 8, 17, 8191, 65543])
+@pytest.mark.parametrize("vocab", [1, 7, 8, 17, 8191, 65535, 65543])
 @pytest.mark.parametrize("kind", ["randn", "zeros", "ties", "nan", "-inf"])
 def test_argmax_edges(ops, dev, vocab, kind):
     """Rows that start 2 to 14 bytes past a 16-byte boundary, single elements
