@@ -153,19 +153,19 @@ class Q4_0LinearMethod(_Base):
         elif m == 1:
             out = torch_ops.q4_0_gemv(rows, w, n, k)
         elif m <= GEMM_MAX_ROWS and k % 64 == 0:
-            out = torch_ops.q4_0_gemm(_aligned16(rows), gemm_weight(layer), n, k)
+            out = torch_ops.q4_0_gemm(aligned16(rows), gemm_weight(layer), n, k)
         elif m <= GEMM_MAX_ROWS and n * k >= GEMM_ROWS_MIN_WEIGHTS and w.data_ptr() % 4 == 0:
             # K % 64 != 0: one launch for all rows (4001 x 2592, 5 rows: 5.5 us;
             # the GEMV below is 5.8 us for each)
-            out = torch_ops.q4_0_gemm_rows(_aligned16(rows), w, n, k)
+            out = torch_ops.q4_0_gemm_rows(aligned16(rows), w, n, k)
         elif m <= GEMM_MAX_ROWS:
             # the GEMV (any K % 32 == 0, 2-byte aligned), one launch per row
             out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
             for i in range(m):
                 torch_ops.q4_0_gemv(rows[i], w, n, k, out=out[i])
         elif (n * k >= GEMM_ROWS_MIN_WEIGHTS and w.data_ptr() % 4 == 0
-              and torch_ops.gemm_rows_preferred(m, n, k) and not _torch_sees(rows)):
-            out = torch_ops.q4_0_gemm_rows(_aligned16(rows), w, n, k)
+              and torch_ops.gemm_rows_preferred(m, n, k) and not torch_sees(rows)):
+            out = torch_ops.q4_0_gemm_rows(aligned16(rows), w, n, k)
         else:
             w_bf16 = torch_ops.q4_0_dequant_bf16(w, n, k)
             out = torch.nn.functional.linear(rows, w_bf16.view(n, k))
@@ -186,12 +186,12 @@ class Q4_0LinearMethod(_Base):
                                           layer.q4_0_k, out=out)
 
 
-def _aligned16(rows: torch.Tensor) -> torch.Tensor:
+def aligned16(rows: torch.Tensor) -> torch.Tensor:
     """The GEMM kernels stage activations in 16-byte chunks."""
     return rows.clone() if rows.data_ptr() % 16 else rows
 
 
-def _torch_sees(rows: torch.Tensor) -> bool:
+def torch_sees(rows: torch.Tensor) -> bool:
     """Whether a product of `rows` has to be a torch operation: autograd or a
     forward-mode level records it, a functorch transform or a tensor subclass
     or mode intercepts it, or autocast chooses its type."""

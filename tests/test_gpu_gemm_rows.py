@@ -142,3 +142,25 @@ def test_linear_routes(dev):
     off = torch.empty(m * k + 1, dtype=torch.bfloat16, device=dev)[1:].view(m, k).copy_(x)
     assert torch.equal(layer(off), y)  # 2-byte aligned rows
     assert torch.equal(layer(off[:5]), layer(x[:5]))
+
+
+@pytest.mark.parametrize("rows", [2, 7, 16, 17])
+def test_head_rows(dev, rows):
+    """2 to 16 rows of logits multiply the exact weights (any 2-D strides and
+    alignment), more the tied bf16 ones, and rows autograd records keep their
+    gradient."""
+    import torch
+    head_mod = pkg("integration.head")
+    vocab, hidden = 1003, 320
+    blocks = oq.make_blocks(vocab, hidden, seed=9)
+    head = head_mod.TiedQ4_0Head(_w(blocks, dev).view(vocab, -1), vocab, hidden)
+    x = randn_bf16(np.random.default_rng(rows), (rows, hidden))
+    xd = bf16_dev(x, dev).view(rows, hidden)
+    y = head.logits(xd)
+    _check(f32_of(y).reshape(rows, vocab), x, _weights(blocks, vocab, hidden, rows))
+    wide = torch.zeros((rows, 2 * hidden + 1), dtype=torch.bfloat16, device=dev)
+    wide[:, 1:hidden + 1] = xd
+    assert torch.equal(head.logits(wide[:, 1:hidden + 1]), y)
+    xg = xd.clone().requires_grad_(True)
+    head.logits(xg).float().sum().backward()
+    assert xg.grad is not None
