@@ -41,6 +41,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef uint32_t u32_a2 __attribute__((aligned(2)));
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 
+// pack_bf16x2 as one v_cvt_pk_bf16_f32 (it compiles to two conversions, shifted
+// and joined); the same bits.  Half of this kernel's operations are conversions.
+__device__ __forceinline__ uint32_t cvt_pk_bf16(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
+
 // 4x4 transpose across the four 16-lane rows: on entry row j of r_g holds
 // X[j][g]; on exit row g of r_k holds X[k][g] (see q4_0_gemm_tile_kernel).
 __device__ __forceinline__ void transpose4(uint32_t& r0, uint32_t& r1, uint32_t& r2,
@@ -83,10 +90,10 @@ __device__ __forceinline__ bf16x8 group_operand(uint32_t lo, uint32_t hi, uint32
         f16x2, perm_b32(0x64646464u, b, (i & 1) ? 0x04030402u : 0x04010400u));
     const f16x2 v = t - f16x2{(_Float16)1032.0f, (_Float16)1032.0f};
     if constexpr (EXACT) {
-      r[i] = pack_bf16x2((float)v[0], (float)v[1]);
+      r[i] = cvt_pk_bf16((float)v[0], (float)v[1]);
     } else {
       const uint32_t vu = __builtin_bit_cast(uint32_t, v);
-      r[i] = pack_bf16x2(mul_mix<false, D_HI>(vu, d), mul_mix<true, D_HI>(vu, d));
+      r[i] = cvt_pk_bf16(mul_mix<false, D_HI>(vu, d), mul_mix<true, D_HI>(vu, d));
     }
   }
   return __builtin_bit_cast(bf16x8, r);
@@ -290,7 +297,7 @@ __global__ __launch_bounds__(64 * WN * WK) void q4_0_gemm_rows_kernel(
           for (int c = 0; c < 4; ++c) s[c] += red[(v * CT + (cq >> 2)) * 64 + l0 + c][row & 3];
         uint16_t* yo = y + (int64_t)mr * n_out + o;
         if (vec) {  // n_out % 4 == 0 and y 8-byte aligned
-          st_agent(reinterpret_cast<u32x2*>(yo), u32x2{pack_bf16x2(s[0], s[1]), pack_bf16x2(s[2], s[3])});
+          st_agent(reinterpret_cast<u32x2*>(yo), u32x2{cvt_pk_bf16(s[0], s[1]), cvt_pk_bf16(s[2], s[3])});
         } else {
 #pragma unroll
           for (int c = 0; c < 4; ++c)

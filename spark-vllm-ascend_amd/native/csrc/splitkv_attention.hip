@@ -103,7 +103,7 @@ __device__ __forceinline__ void norm_rope_head(float a, float b, float ga, float
 }
 
 // The arguments the first loads depend on are passed ahead of the rest as
-// scalars and pointers (15 dwords): the library is built with kernel-argument
+// scalars and pointers (14 dwords): the library is built with kernel-argument
 // preloading, which places leading non-aggregate arguments in SGPRs, so the
 // first loads issue without a kernarg fetch.  pa_ / pb_ are the positions
 // and slots (FUSEQ: the per-sequence gather reads them at entry) or the K and
@@ -117,7 +117,7 @@ template <int WAVES, int BLK, bool FUSEQ, bool PLAN, bool RECFAST = false>
 __global__ __launch_bounds__(64 * WAVES) __attribute__((amdgpu_waves_per_eu(PLAN ? 2 : 1)))
 void splitkv_decode_kernel(
     const int32_t* block_table_, const void* lens_, const void* pa_, const void* pb_,
-    const uint16_t* q_, int num_splits_, int max_blocks_, int bs_log2_, int n_kv_, int probe_,
+    const uint16_t* q_, int num_splits_, int max_blocks_, int bs_log2_, int n_kv_,
     SplitKVArgs A) {
   A.block_table = block_table_;
   A.seq_lens = (const int32_t*)lens_;
@@ -131,7 +131,10 @@ void splitkv_decode_kernel(
   A.q = q_;
   A.num_splits = num_splits_;
   A.max_blocks = max_blocks_;
-  A.bs_log2 = bs_log2_;
+  // a plan's launch carries its probe record (plus 1) above the block size, as
+  // more arguments than 14 dwords are not preloaded
+  A.bs_log2 = PLAN ? bs_log2_ & 0xff : bs_log2_;
+  const int probe = PLAN ? (bs_log2_ >> 8) - 1 : -1;
   A.n_kv = n_kv_;
   A.n_q = 4 * n_kv_;  // GQA 4:1 (validated on the host)
   static_assert(BLK == 32 || BLK == 64, "blocks of 32 or 64 tokens");
@@ -183,7 +186,7 @@ void splitkv_decode_kernel(
   bool pos_ok = true;  // FUSEQ: a position and a slot come with the split
   if constexpr (PLAN) {
     gv = reinterpret_cast<const uint32_t*>(
-        lens_)[lane == PROBE_LANE ? (int64_t)max(probe_, 0) * PLAN_WORDS
+        lens_)[lane == PROBE_LANE ? (int64_t)max(probe, 0) * PLAN_WORDS
                                   : (int64_t)rec * PLAN_WORDS + lane];
     seq = __builtin_amdgcn_readlane((int)gv, 0);
     if (seq < 0) return;  // an unused record: the plan cleared the unused partials
@@ -194,7 +197,7 @@ void splitkv_decode_kernel(
     pos_ok = (w3 & PLAN_HAS_POSITIONS) != 0;
     // waves with blocks (lane PROBE_LANE: the sequence of the record that is in
     // use from PLAN_ONE_WAVE_WGS live workgroups on)
-    const bool many = probe_ >= 0 && __builtin_amdgcn_readlane((int)gv, PROBE_LANE) >= 0;
+    const bool many = probe >= 0 && __builtin_amdgcn_readlane((int)gv, PROBE_LANE) >= 0;
     const int active = many && s_end - s0 >= PLAN_ONE_WAVE_TOKENS ? 1 : WAVES;
     w0 = wave < active ? min(s0 + wave * BLK, s_end) : s_end;
     step = active * BLK;
@@ -784,6 +787,7 @@ int launch_splitkv(void* stream, smx::SplitKVArgs a, int32_t num_seqs, int32_t b
   // the record in use from PLAN_ONE_WAVE_WGS live workgroups on (-1: there is none)
   const int last_few = (smx::PLAN_ONE_WAVE_WGS - 1) / a.n_kv;
   const int probe = plan && last_few < num_records ? last_few : -1;
+  const int bs_arg = a.bs_log2 | ((probe + 1) << 8);  // without a plan the block size alone
 #define SMX_ATTN_LAUNCH(W, B)                                                                   \
   do {                                                                                          \
     if (plan && recfast)                                                                        \
@@ -791,19 +795,19 @@ int launch_splitkv(void* stream, smx::SplitKVArgs a, int32_t num_seqs, int32_t b
                          dim3(64 * W), 0, (hipStream_t)stream, a.block_table, (const void*)plan,  \
                          FUSEQ ? (const void*)a.positions : (const void*)a.kc,                     \
                          FUSEQ ? (const void*)a.slot_mapping : (const void*)a.vc, a.q,             \
-                         a.num_splits, a.max_blocks, a.bs_log2, a.n_kv, probe, a);                        \
+                         a.num_splits, a.max_blocks, bs_arg, a.n_kv, a);                        \
     else if (plan)                                                                              \
       SMX_LAUNCH((smx::splitkv_decode_kernel<W, B, FUSEQ, true>), grid, dim3(64 * W),   \
                          0, (hipStream_t)stream, a.block_table, (const void*)plan,                \
                          FUSEQ ? (const void*)a.positions : (const void*)a.kc,                     \
                          FUSEQ ? (const void*)a.slot_mapping : (const void*)a.vc, a.q,             \
-                         a.num_splits, a.max_blocks, a.bs_log2, a.n_kv, probe, a);                        \
+                         a.num_splits, a.max_blocks, bs_arg, a.n_kv, a);                        \
     else                                                                                        \
       SMX_LAUNCH((smx::splitkv_decode_kernel<W, B, FUSEQ, false>), grid, dim3(64 * W),  \
                          0, (hipStream_t)stream, a.block_table, (const void*)a.seq_lens,          \
                          FUSEQ ? (const void*)a.positions : (const void*)a.kc,                     \
                          FUSEQ ? (const void*)a.slot_mapping : (const void*)a.vc, a.q,             \
-                         a.num_splits, a.max_blocks, a.bs_log2, a.n_kv, probe, a);                        \
+                         a.num_splits, a.max_blocks, bs_arg, a.n_kv, a);                        \
   } while (0)
   if (blk == 32) {
     if (waves == 8) SMX_ATTN_LAUNCH(8, 32);
