@@ -56,15 +56,6 @@ constexpr int PLAN_WORDS = 64;
 constexpr int PLAN_PAGE0 = 9;
 constexpr int PLAN_ALIGN = 128;  // split lengths are multiples of this (4 waves x 32 tokens)
 constexpr uint32_t PLAN_HAS_POSITIONS = 0x80000000u;  // word 3 flag
-// One wave of a workgroup walks the whole of a split of PLAN_ONE_WAVE_TOKENS or
-// more where the live records make PLAN_ONE_WAVE_WGS workgroups or more: those
-// alone, 16 KB of loads each, keep HBM busy, and more waves only add streams that
-// get in each other's way (8 sequences to 32768 tokens, 545 MB: 4 waves 125 us,
-// 1 wave 113; to 16384: 67.6, 64.3; 16 to 8192: 104.4, 102.1).  With fewer or
-// shorter splits the waves share the latency (6 sequences to 16384: 50.9, 1 wave
-// 61.7; 16 to 1024: 19.3, 20.6).
-constexpr int PLAN_ONE_WAVE_WGS = 512;
-constexpr int PLAN_ONE_WAVE_TOKENS = 768;
 
 struct SplitKVArgs {
   const uint16_t* q;  // [num_seqs, n_q, HD] (plain) or the raw QKV row (FUSEQ)
@@ -131,10 +122,7 @@ void splitkv_decode_kernel(
   A.q = q_;
   A.num_splits = num_splits_;
   A.max_blocks = max_blocks_;
-  // a plan's launch carries its probe record (plus 1) above the block size, as
-  // more arguments than 14 dwords are not preloaded
-  A.bs_log2 = PLAN ? bs_log2_ & 0xff : bs_log2_;
-  const int probe = PLAN ? (bs_log2_ >> 8) - 1 : -1;
+  A.bs_log2 = bs_log2_;
   A.n_kv = n_kv_;
   A.n_q = 4 * n_kv_;  // GQA 4:1 (validated on the host)
   static_assert(BLK == 32 || BLK == 64, "blocks of 32 or 64 tokens");
@@ -177,17 +165,12 @@ void splitkv_decode_kernel(
   // not from the length, so all of it is one round trip; a plan record holds
   // the bounds and the first pages itself.
   constexpr int PB = PLAN ? PLAN_PAGE0 : 8;  // lane of the first gathered page
-  constexpr int PROBE_LANE = 63;         // plan: not a page but the word described below
-  constexpr int PEND = PLAN ? PROBE_LANE : 64;  // end of the gathered pages
   constexpr int LEN_LANE = PLAN ? 4 : 0, POS_LANE = PLAN ? 5 : 3, SLOT_LANE = PLAN ? 7 : 5;
   uint32_t gv;
-  int seq, split, s0, s_end, wlen = 0, w0, pg0;
-  int step = BLK;  // tokens from a wave's block to its next
+  int seq, split, s0, s_end, wlen, w0, pg0;
   bool pos_ok = true;  // FUSEQ: a position and a slot come with the split
   if constexpr (PLAN) {
-    gv = reinterpret_cast<const uint32_t*>(
-        lens_)[lane == PROBE_LANE ? (int64_t)max(probe, 0) * PLAN_WORDS
-                                  : (int64_t)rec * PLAN_WORDS + lane];
+    gv = reinterpret_cast<const uint32_t*>(lens_)[(int64_t)rec * PLAN_WORDS + lane];
     seq = __builtin_amdgcn_readlane((int)gv, 0);
     if (seq < 0) return;  // an unused record: the plan cleared the unused partials
     s0 = __builtin_amdgcn_readlane((int)gv, 1);
@@ -195,12 +178,8 @@ void splitkv_decode_kernel(
     const uint32_t w3 = (uint32_t)__builtin_amdgcn_readlane((int)gv, 3);
     split = (int)(w3 & ~PLAN_HAS_POSITIONS);
     pos_ok = (w3 & PLAN_HAS_POSITIONS) != 0;
-    // waves with blocks (lane PROBE_LANE: the sequence of the record that is in
-    // use from PLAN_ONE_WAVE_WGS live workgroups on)
-    const bool many = probe >= 0 && __builtin_amdgcn_readlane((int)gv, PROBE_LANE) >= 0;
-    const int active = many && s_end - s0 >= PLAN_ONE_WAVE_TOKENS ? 1 : WAVES;
-    w0 = wave < active ? min(s0 + wave * BLK, s_end) : s_end;
-    step = active * BLK;
+    wlen = ((s_end - s0 + WAVES - 1) / WAVES + TILE - 1) / TILE * TILE;
+    w0 = min(s0 + wave * wlen, s_end);
     pg0 = s0 >> bs_log2;
   } else {
     split = blockIdx.y;
@@ -261,7 +240,7 @@ void splitkv_decode_kernel(
   // covers t, else a block-table load
   auto page_of = [&](int t) -> int {
     const int li = (t >> bs_log2) - pg0 + PB;
-    return li < PEND ? (int)lane_u32(li) : bt[min(t >> bs_log2, max_blocks - 1)];
+    return li < 64 ? (int)lane_u32(li) : bt[min(t >> bs_log2, max_blocks - 1)];
   };
   // the first two pages: with capacity splits always gathered (lanes PB and
   // PB or PB + 1: no branch), with a plan maybe past the record
@@ -283,7 +262,7 @@ void splitkv_decode_kernel(
     stores_done();
     return;
   }
-  const int w1 = PLAN ? s1 : min(s1, w0 + wlen);
+  const int w1 = min(s1, w0 + wlen);
 
   const int bs = 1 << bs_log2;
   const int64_t tok_stride = (int64_t)n_kv * HD;
@@ -409,7 +388,7 @@ void splitkv_decode_kernel(
   for (int t = 0; t < 8; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
   uint16_t* pw = reinterpret_cast<uint16_t*>(p2[wave]);  // P as bf16 [head G][BLK]
 
-  for (int t0 = w0; t0 < w1; t0 += step) {
+  for (int t0 = w0; t0 < w1; t0 += BLK) {
     if (t0 != w0) load_block(t0);
 
     if constexpr (FUSEQ) {
@@ -760,13 +739,13 @@ int launch_splitkv(void* stream, smx::SplitKVArgs a, int32_t num_seqs, int32_t b
   const int64_t tps = ((cap + a.num_splits - 1) / a.num_splits + 31) / 32 * 32;
   int blk = tps <= 256 ? 32 : 64;
   int waves = blk == 64 ? 8 : tps <= 32 ? 1 : tps <= 64 ? 2 : tps <= 128 ? 4 : 8;
-  // With a plan 4 waves of 32-token blocks per workgroup, taking the split's
-  // blocks in turn (2 waves are up to 18 % slower from 2 to 32
-  // sequences to 256..16384 tokens, 8 waves slower but for a few long sequences;
-  // 64-token blocks take 246 VGPRs), or one taking all (PLAN_ONE_WAVE_WGS).
+  // A plan's splits are long (the batch's tokens over a few hundred
+  // workgroups): 2 waves of 32-token blocks per workgroup, each wave half a
+  // split (8-sequence step: 2 waves 4.69-4.72 ms, 4 waves 4.72-4.74, 1 wave
+  // 5.06; 64-token blocks take 246 VGPRs and measured 5.02).
   if (plan) {
     blk = 32;
-    waves = 4;
+    waves = 2;
   }
   const char* e = smx::tuning_env("SMX_ATTN_WAVES");  // "waves[,blk]" override for tuning sweeps
   if (e) {
@@ -784,10 +763,6 @@ int launch_splitkv(void* stream, smx::SplitKVArgs a, int32_t num_seqs, int32_t b
   const bool recfast = plan && num_records % 8 == 0;
   const dim3 grid = plan ? (recfast ? dim3(num_records, a.n_kv, 1) : dim3(a.n_kv, num_records, 1))
                          : dim3(a.n_kv, a.num_splits, num_seqs);
-  // the record in use from PLAN_ONE_WAVE_WGS live workgroups on (-1: there is none)
-  const int last_few = (smx::PLAN_ONE_WAVE_WGS - 1) / a.n_kv;
-  const int probe = plan && last_few < num_records ? last_few : -1;
-  const int bs_arg = a.bs_log2 | ((probe + 1) << 8);  // without a plan the block size alone
 #define SMX_ATTN_LAUNCH(W, B)                                                                   \
   do {                                                                                          \
     if (plan && recfast)                                                                        \
@@ -795,19 +770,19 @@ int launch_splitkv(void* stream, smx::SplitKVArgs a, int32_t num_seqs, int32_t b
                          dim3(64 * W), 0, (hipStream_t)stream, a.block_table, (const void*)plan,  \
                          FUSEQ ? (const void*)a.positions : (const void*)a.kc,                     \
                          FUSEQ ? (const void*)a.slot_mapping : (const void*)a.vc, a.q,             \
-                         a.num_splits, a.max_blocks, bs_arg, a.n_kv, a);                        \
+                         a.num_splits, a.max_blocks, a.bs_log2, a.n_kv, a);                        \
     else if (plan)                                                                              \
       SMX_LAUNCH((smx::splitkv_decode_kernel<W, B, FUSEQ, true>), grid, dim3(64 * W),   \
                          0, (hipStream_t)stream, a.block_table, (const void*)plan,                \
                          FUSEQ ? (const void*)a.positions : (const void*)a.kc,                     \
                          FUSEQ ? (const void*)a.slot_mapping : (const void*)a.vc, a.q,             \
-                         a.num_splits, a.max_blocks, bs_arg, a.n_kv, a);                        \
+                         a.num_splits, a.max_blocks, a.bs_log2, a.n_kv, a);                        \
     else                                                                                        \
       SMX_LAUNCH((smx::splitkv_decode_kernel<W, B, FUSEQ, false>), grid, dim3(64 * W),  \
                          0, (hipStream_t)stream, a.block_table, (const void*)a.seq_lens,          \
                          FUSEQ ? (const void*)a.positions : (const void*)a.kc,                     \
                          FUSEQ ? (const void*)a.slot_mapping : (const void*)a.vc, a.q,             \
-                         a.num_splits, a.max_blocks, bs_arg, a.n_kv, a);                        \
+                         a.num_splits, a.max_blocks, a.bs_log2, a.n_kv, a);                        \
   } while (0)
   if (blk == 32) {
     if (waves == 8) SMX_ATTN_LAUNCH(8, 32);

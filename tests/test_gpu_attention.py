@@ -340,10 +340,10 @@ def test_backend_forward(dev, planned):
 
 
 @pytest.mark.parametrize("fused", [False, True])
-def test_plan_one_wave_per_workgroup(ops, dev, fused):
-    """At least 512 live workgroups and splits of 768 tokens: one wave walks a
-    split (70 items here; 40 are just below, four waves): against capacity
-    splits of the same inputs, the new token's K/V included."""
+def test_plan_of_many_workgroups(ops, dev, fused):
+    """Plans of more and of fewer than 512 live workgroups (70 and 40 items,
+    splits of 768 tokens and more) against capacity splits of the same inputs,
+    the new token's K/V included."""
     import torch
     att = pkg("integration.attention")
     n_kv, n_q, hd, bs, splits = 8, 32, 128, 128, 32
@@ -358,7 +358,7 @@ def test_plan_one_wave_per_workgroup(ops, dev, fused):
     slots = table[torch.arange(S, device=dev), pos // bs].long() * bs + pos % bs
     scale = hd ** -0.5
     outs, caches = [], []
-    for items in (0, 40, 70):  # capacity splits, 4 waves, 1 wave
+    for items in (0, 40, 70):  # 0: capacity splits
         c = kv.clone()
         po, pl = att.split_partials(S, splits, n_q, hd, dev)
         plan = None
@@ -393,3 +393,32 @@ def test_plan_one_wave_per_workgroup(ops, dev, fused):
         # bf16 probabilities at other running maxima: 2^-8 of the output's own size
         torch.testing.assert_close(o, outs[0], rtol=2.0 ** -6, atol=2.0 ** -6 * float(outs[0].std()))
         assert torch.equal(c, caches[0])
+
+
+def test_plan_result_independent_of_other_sequences(ops, dev):
+    """A sequence split at the same tokens gives the same bits alone (136
+    workgroups) and among three others (544): the order of a split's sums and
+    the maxima its bf16 probabilities are taken at follow from the split."""
+    import torch
+    att = pkg("integration.attention")
+    bs, splits, items, per_seq = 128, 20, 70, 104
+    lens = [12801, 12700, 12600, 12500]  # splits of 768 tokens, from the first length
+    g = torch.Generator(device=dev)
+    g.manual_seed(11)
+    table = torch.randperm(len(lens) * per_seq, generator=g, device=dev).to(torch.int32)
+    table = table.view(len(lens), per_seq)
+    kc, vc = torch.randn((2, len(lens) * per_seq, bs, N_KV, HD), generator=g,
+                         device=dev).to(torch.bfloat16)
+    q = torch.randn((len(lens), N_Q, HD), generator=g, device=dev).to(torch.bfloat16)
+    outs = []
+    for n in (1, len(lens)):
+        L = torch.tensor(lens[:n], dtype=torch.int32, device=dev)
+        po, pl = att.split_partials(n, splits, N_Q, HD, dev)
+        plan = ops.splitkv_plan(L, table[:n], bs, items, po, pl)
+        live = plan[plan[:, 0] >= 0]
+        assert live.shape[0] == (17 if n == 1 else 68)
+        assert int((live[:, 2] - live[:, 1]).max()) == 768
+        out = ops.splitkv_decode_planned_merged(q[:n], kc, vc, table[:n], plan, items, HD ** -0.5,
+                                                po, pl)
+        outs.append(out[0].clone())
+    assert torch.equal(outs[0], outs[1])
