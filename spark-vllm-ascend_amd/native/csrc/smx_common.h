@@ -55,9 +55,10 @@ __device__ __forceinline__ void st_agent(u32x4* p, u32x4 v) {  // two 64-bit sto
 //  * agent_rsrc + st_agent_b128(r, off, v): a raw buffer store with the sc1
 //    cache policy, at byte offset off from the wave-uniform base of r; lanes
 //    at or past r's byte count store nothing;
-//  * st_agent_b128(p, v): any 16-byte aligned address per lane.  The s_nop is
-//    the wait state a store of more than 64 bits needs before its data
-//    registers are overwritten, which the compiler does not add after an asm.
+//  * st_agent_b128(p, v): any 16-byte aligned address per lane.  s_nop 1 is the
+//    two wait states that gfx940 and later need between a store of more than 64
+//    bits and a VALU write to its data registers; the compiler adds them (as
+//    s_nop 1) to its own stores, but not after an asm.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t agent_rsrc(void* base, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(base, 0, (int)bytes, 0x00027000);
 }
@@ -66,7 +67,7 @@ __device__ __forceinline__ void st_agent_b128(__amdgpu_buffer_rsrc_t r, uint32_t
   __builtin_amdgcn_raw_buffer_store_b128(v, r, (int)off, 0, SC1);
 }
 __device__ __forceinline__ void st_agent_b128(void* p, u32x4 v) {
-  __asm__ volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v) : "memory");
+  __asm__ volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(p), "v"(v) : "memory");
 }
 __device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0); }
 

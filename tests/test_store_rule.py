@@ -5,7 +5,12 @@ store to an s_endpgm there is a full wait (s_waitcnt vmcnt(0): on gfx9
 targets vmcnt counts stores too).  Read from the AMD disassembly of the code
 objects this repository builds; the scan follows branches (s_branch,
 s_cbranch_*), so a store in a block that jumps to a shared s_endpgm is
-checked on that path too."""
+checked on that path too.
+
+Also checked: a vector-memory store of more than 64 bits reads its data
+registers late, so on this target two wait states separate it from a VALU
+write to them.  The compiler inserts them for its own stores; the stores
+written as inline asm carry their own s_nop."""
 import functools
 import re
 import shutil
@@ -108,6 +113,52 @@ def unwaited_ends(funcs: dict) -> tuple:
     return ends, late
 
 
+WIDE = re.compile(r"^(global|flat|buffer|scratch)_store_(dwordx[34]|b96|b128)\b")
+STORE_WAIT_STATES = 2
+
+
+def _vgprs(operand: str) -> set:
+    m = re.fullmatch(r"v(\d+)|v\[(\d+):(\d+)\]", operand)
+    if not m:
+        return set()
+    lo = int(m.group(1) or m.group(2))
+    return set(range(lo, int(m.group(3) or lo) + 1))
+
+
+def _operands(ins: str) -> list:
+    return [o.split()[0] for o in ins.partition(" ")[2].split(",") if o.strip()]
+
+
+def wide_stores(lines) -> list:
+    """(index, data registers) of the stores of more than 64 bits."""
+    return [(i, _vgprs(_operands(ins)[0 if ins.startswith("buffer") else 1]))
+            for i, (_, ins, _) in enumerate(lines) if WIDE.match(ins)]
+
+
+def overwritten_store_data(funcs: dict) -> list:
+    """(kernel, store, instruction) wherever a VALU instruction fewer than
+    STORE_WAIT_STATES wait states after a wide store writes its data."""
+    bad = []
+    for name, lines in funcs.items():
+        index = {addr: i for i, (addr, _, _) in enumerate(lines)}
+        for i, data in wide_stores(lines):
+            work = [(j, 0) for j in _successors(lines, i, index)]
+            while work:
+                j, waited = work.pop()
+                if waited >= STORE_WAIT_STATES:
+                    continue
+                ins = lines[j][1]
+                if ins.startswith("v_"):
+                    ops = _operands(ins)
+                    both = "swap" in ins.split()[0]  # exchanges its two operands
+                    if data & set().union(*map(_vgprs, ops[:2 if both else 1])):
+                        bad.append((name, lines[i][1], ins))
+                        continue
+                waited += int(ins.split()[1], 0) + 1 if ins.startswith("s_nop") else 1
+                work += [(k, waited) for k in _successors(lines, j, index)]
+    return bad
+
+
 def _lines(*ins):
     """Planted kernels: instructions at 4-byte addresses, "-> k" marking a
     branch to instruction k."""
@@ -169,3 +220,39 @@ def test_stores_complete_before_every_kernel_end():
         late += [(path.name, n[:80]) for n in l]
     assert ends > 100
     assert not late, f"a store not waited for before s_endpgm on some path: {late[:5]}"
+
+
+def test_the_wait_state_scan_finds_planted_mistakes():
+    st = "global_store_dwordx4 v[4:5], v[6:9], off sc1"
+    funcs = {"ok": _lines(st, "s_nop 1", "v_mov_b32_e32 v6, 0", "s_endpgm"),
+             "short": _lines(st, "s_nop 0", "v_mov_b32_e32 v9, 0", "s_endpgm"),
+             "scalars": _lines(st, "s_add_u32 s0, s0, 1", "s_nop 0", "v_mov_b32_e32 v6, 0",
+                               "s_endpgm"),
+             "other": _lines(st, "v_mov_b32_e32 v10, 0", "v_add_f32_e32 v4, v6, v7", "s_endpgm"),
+             "narrow": _lines("global_store_dwordx2 v[4:5], v[6:7], off sc1",
+                              "v_mov_b32_e32 v6, 0", "s_endpgm"),
+             "branch": _lines(st, "s_branch -> 3", "s_endpgm", "v_mov_b32_e32 v[7:8], 0",
+                              "s_endpgm"),
+             "swap": _lines("buffer_store_dwordx4 v[0:3], v4, s[0:3], 0 offen sc1",
+                            "v_permlane32_swap_b32_e32 v8, v3", "s_endpgm")}
+    assert sorted(n for n, _, _ in overwritten_store_data(funcs)) == ["branch", "short", "swap"]
+
+
+def test_wide_stores_keep_their_data():
+    """Two wait states on every path, and right behind each store written as
+    inline asm (the 16-byte global stores), whatever is scheduled after it."""
+    bare, bad, count = [], [], 0
+    for path in _code_objects():
+        funcs = _disassemble(path)
+        bad += [(path.name, n[:80], s, i) for n, s, i in overwritten_store_data(funcs)]
+        for name, lines in funcs.items():
+            for i, _ in wide_stores(lines):
+                if lines[i][1].startswith("global_store_dwordx4"):
+                    count += 1
+                    nxt = lines[i + 1][1]
+                    if not (nxt.startswith("s_nop")
+                            and int(nxt.split()[1], 0) + 1 >= STORE_WAIT_STATES):
+                        bare.append((path.name, name[:80], lines[i][1], nxt))
+    assert count > 0
+    assert not bad, f"store data overwritten too early: {bad[:5]}"
+    assert not bare, f"asm stores without two wait states of their own: {bare[:5]}"
