@@ -54,6 +54,8 @@ class TiedQ4_0Head(torch.nn.Module):
         return torch_ops.embedding(self.weight, ids, out=out)
 
 
-def greedy_sample(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
-    """argmax over the vocabulary (temperature 0), lowest index on ties."""
-    return torch_ops.argmax(logits, out=out)
+def greedy_sample(logits: torch.Tensor, out: torch.Tensor | None = None,
+                  keys: torch.Tensor | None = None) -> torch.Tensor:
+    """argmax over the vocabulary (temperature 0), lowest index on ties; keys:
+    torch_ops.argmax's workspace."""
+    return torch_ops.argmax(logits, out=out, keys=keys)

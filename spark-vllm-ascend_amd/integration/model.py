@@ -230,6 +230,10 @@ class DecodeModel:
               else torch_ops.gemm_keys_per_row(c.vocab))
         self.argmax_keys = (torch.empty((B, nk), dtype=torch.int64, device=dev) if nk > 0
                             else None)
+        # where the step ends in an argmax launch of its own: that one's workspace
+        nk = torch_ops.argmax_num_keys(B, c.vocab)
+        self.sample_keys = (torch.empty((nk,), dtype=torch.int64, device=dev)
+                            if nk > 0 and not self.fused and B == 1 else None)
         self.graph: torch.cuda.CUDAGraph | None = None
         self.runner = None  # native.runner.StepRunner after record_runner()
 
@@ -353,7 +357,7 @@ class DecodeModel:
             ops.add_rmsnorm(x_in, r_in, self.final_norm, c.eps, out=self.h,
                             residual_out=self.res_a)
             ops.q4_0_gemv(self.h, self.head.q4_0_head, c.vocab, c.hidden, out=self.logits)
-            ops.argmax(self.logits, out=st.next_ids)
+            ops.argmax(self.logits, out=st.next_ids, keys=self.sample_keys)
         ops.decode_advance(st.next_ids, st.ids, st.positions, st.seq_lens, st.slot_mapping,
                            st.block_table, c.block_size, tokens_out=st.tokens,
                            forced_ids=st.forced, forced_len=st.forced_len, argmax_keys=keys,

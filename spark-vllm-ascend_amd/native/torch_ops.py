@@ -348,18 +348,31 @@ def embedding(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor | None =
     return out
 
 
-def argmax(logits: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+def argmax_num_keys(rows: int, vocab: int) -> int:
+    """Elements of the `keys` workspace argmax() takes; 0 where it uses none."""
+    return rows * load().smx_argmax_parts(vocab) if 1 <= rows <= 65535 else 0
+
+
+def argmax(logits: torch.Tensor, out: torch.Tensor | None = None,
+           keys: torch.Tensor | None = None) -> torch.Tensor:
+    """Greedy token of each row.  Long rows take two launches with a workspace
+    between them: `keys` (int64, argmax_num_keys elements), else one allocated
+    here.  With `out` and no `keys` the call allocates nothing, as a recorded
+    step must not, and the row takes one launch."""
     _check(logits, "logits", BF16)
     vocab = logits.shape[-1]
     rows = logits.numel() // vocab
+    num_keys = argmax_num_keys(rows, vocab)
+    if keys is not None:
+        _check(keys, "keys", torch.int64, num_keys, logits.device)
+    elif num_keys and out is None:
+        keys = torch.empty((num_keys,), dtype=torch.int64, device=logits.device)
     if out is None:
         out = torch.empty((rows,), dtype=torch.int64, device=logits.device)
     _check(out, "out", torch.int64, rows, logits.device)
-    parts = load().smx_argmax_parts(vocab) if 1 <= rows <= 65535 else 0
-    if parts:
-        keys = torch.empty((rows, parts), dtype=torch.int64, device=logits.device)
+    if num_keys and keys is not None:
         call("smx_argmax_bf16_parts", _stream(logits), logits.data_ptr(), rows, vocab,
-             keys.data_ptr(), rows * parts, out.data_ptr())
+             keys.data_ptr(), num_keys, out.data_ptr())
         return out
     call("smx_argmax_bf16", _stream(logits), logits.data_ptr(), rows, vocab, out.data_ptr())
     return out

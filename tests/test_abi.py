@@ -73,6 +73,12 @@ def test_bindings_cover_header():
     ("smx_silu_mul", (None, 16, 16, 0, 10)),
     ("smx_embedding", (None, 16, 16, 16, 0, 10, 10)),
     ("smx_argmax_bf16", (None, 16, 0, 10, 16)),
+    ("smx_argmax_bf16_parts", (None, 16, 0, 151936, 16, 0, 16)),
+    ("smx_argmax_bf16_parts", (None, 16, 65536, 151936, 16, 65536 * 32, 16)),
+    ("smx_argmax_bf16_parts", (None, 16, 2, 151936, 16, 32, 16)),
+    ("smx_argmax_bf16_parts", (None, 16, 1, 1000, 16, 0, 16)),
+    ("smx_argmax_bf16_parts", (None, 16, 1, 151936, 12, 32, 16)),
+    ("smx_argmax_bf16_parts", (None, 16, 1, 151936, None, 32, 16)),
     ("smx_decode_advance", (None, 16, None, 0, None, None, 16, 16, 16, 16, 16, None, 0, 1, 1, 0, None, None, 0, 0)),
     ("smx_decode_advance", (None, 16, None, 0, None, 16, 16, 16, 16, 16, 16, None, 1, 1, 1, 0, None, None, 0, 0)),
     ("smx_decode_advance", (None, 16, None, 0, 16, 16, 16, 16, 16, 16, 16, None, 1, 1, 1, 0, None, None, 0, 0)),

@@ -27,9 +27,9 @@ def _m():
     return pkg("integration.model")
 
 
-def tiny_cfg(activation="swiglu"):
+def tiny_cfg(activation="swiglu", vocab=1000):
     return _m().DecoderConfig(hidden=256, n_layers=2, n_q=8, n_kv=2, head_dim=128,
-                              intermediate=512, vocab=1000, block_size=32, activation=activation)
+                              intermediate=512, vocab=vocab, block_size=32, activation=activation)
 
 
 def _state_bits(model):
@@ -50,14 +50,14 @@ def _assert_same(a, b, what):
 
 
 def _eager_vs_runner(dev, fences, *, fused=True, batch=1, steps=30, chunks=(30,), seed=5,
-                     activation="swiglu"):
+                     activation="swiglu", vocab=1000):
     import torch
     m = _m()
     kw = dict(seed=seed, max_len=64, num_splits=2, fused=fused)
     if batch > 1:
         kw.update(batch=batch)
-    e = m.DecodeModel(tiny_cfg(activation), dev, **kw)
-    r = m.DecodeModel(tiny_cfg(activation), dev, **kw)
+    e = m.DecodeModel(tiny_cfg(activation, vocab), dev, **kw)
+    r = m.DecodeModel(tiny_cfg(activation, vocab), dev, **kw)
     rng = np.random.default_rng(seed)
     prompts = [torch.tensor(rng.integers(0, 1000, 3 + i)) for i in range(batch)]
     prompt = prompts[0] if batch == 1 else prompts
@@ -100,6 +100,40 @@ def test_runner_replays_the_gelu_model(dev, fused, batch):
     recorded kernel argument) in the fused, unfused and batched steps."""
     _eager_vs_runner(dev, "acquire", fused=fused, batch=batch, chunks=(10, 20), seed=8,
                      activation="gelu")
+
+
+@pytest.mark.parametrize("fused,batch", [(True, 1), (False, 1), (False, 2)])
+def test_runner_records_a_long_vocabulary(dev, fused, batch):
+    """The step's argmax of rows that smx_argmax_parts splits (the unfused step
+    has it as launches of its own)."""
+    assert pkg("native.torch_ops").argmax_num_keys(1, 151936) > 0
+    _eager_vs_runner(dev, "acquire", fused=fused, batch=batch, chunks=(10, 20), seed=9,
+                     vocab=151936)
+
+
+def test_runner_records_argmax_with_its_outputs(dev):
+    """argmax with a preallocated output, and with a workspace too, records and
+    replays on what the logits hold then; without either it is refused."""
+    import torch
+    ops = pkg("native.torch_ops")
+    StepRunner = pkg("native.runner").StepRunner
+    rows, vocab = 3, 151937
+    logits = torch.randn(rows, vocab, device=dev).to(torch.bfloat16)
+    out = torch.empty(rows, dtype=torch.int64, device=dev)
+    keys = torch.empty(ops.argmax_num_keys(rows, vocab), dtype=torch.int64, device=dev)
+    with StepRunner() as runner:
+        with pytest.raises(RuntimeError, match="allocated"):
+            runner.record(lambda: ops.argmax(logits))
+        for kw, packets in (({}, 1), ({"keys": keys}, 2)):
+            assert runner.record(lambda: ops.argmax(logits, out=out, **kw)) == packets
+            for first in (40000, 7):
+                logits[:, first] = 100.0 + 8 * (40000 - first) / 40000
+                out.fill_(-1)
+                runner.run(2)
+                assert out.tolist() == [first] * rows
+            logits.copy_(torch.randn(rows, vocab, device=dev))
+    with pytest.raises(ValueError, match="keys"):
+        ops.argmax(logits, out=out, keys=keys[1:])
 
 
 @pytest.mark.parametrize("fences", FENCES)
