@@ -392,7 +392,8 @@ int smx_argmax_bf16(void* stream, const void* logits, int64_t rows,
 /*
  * smx_argmax_bf16 by two launches with a workspace between them: keys
  * [rows, smx_argmax_parts(vocab)] uint64, num_keys their number.  The faster way
- * where smx_argmax_parts is not 0 (a row is then too long for one workgroup).
+ * for up to 32 rows where smx_argmax_parts is not 0 (a row is then too long for
+ * one workgroup); more rows fill the chip with a workgroup each.
  */
 int64_t smx_argmax_parts(int64_t vocab);
 int smx_argmax_bf16_parts(void* stream, const void* logits, int64_t rows, int64_t vocab,

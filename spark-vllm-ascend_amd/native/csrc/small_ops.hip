@@ -764,7 +764,8 @@ extern "C" int smx_argmax_bf16(void* stream, const void* logits, int64_t rows, i
 }
 
 extern "C" int64_t smx_argmax_parts(int64_t vocab) {
-  // From 64K elements on; one workgroup takes 7.0 us for 50000, the two launches 6.
+  // From 64K elements on, for few rows: one workgroup takes 7.0 us for 50000, the
+  // two launches 6; for 65536 7.7 and 5.3, 151936 9.1 to 11.1 and 5.9.
   if (vocab < 65536 || vocab > 0xffffffffll) return 0;
   const int64_t len = ((vocab + smx::ARGMAX_PARTS - 1) / smx::ARGMAX_PARTS + 7) / 8 * 8;
   return (vocab + len - 1) / len;

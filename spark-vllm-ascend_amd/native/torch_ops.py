@@ -348,16 +348,27 @@ def embedding(table: torch.Tensor, ids: torch.Tensor, out: torch.Tensor | None =
     return out
 
 
+#: rows up to which the two-launch argmax is the faster one: more rows fill the
+#: chip with one workgroup each (vocab 65536 / 151936 in a graph, two launches
+#: against one: 32 rows 8.1 / 9.2 us, 8.4 / 11.9; 64 rows 10.7 / 12.6, 8.5 / 12.3;
+#: 256 rows 26.9 / 31.9, 9.5 / 19.5)
+ARGMAX_PARTS_ROWS = 32
+#: vocab above which it is also for a call that allocates the keys, about 2.5 us of
+#: the host's time (eager, one row, allocating against one launch: 65536 8.4 us, 7.3;
+#: 98304 8.5, 7.6; 110000 8.6, 9.2; 151936 8.3, 8.8)
+ARGMAX_ALLOC_VOCAB = 98304
+
+
 def argmax_num_keys(rows: int, vocab: int) -> int:
     """Elements of the `keys` workspace argmax() takes; 0 where it uses none."""
-    return rows * load().smx_argmax_parts(vocab) if 1 <= rows <= 65535 else 0
+    return rows * load().smx_argmax_parts(vocab) if 1 <= rows <= ARGMAX_PARTS_ROWS else 0
 
 
 def argmax(logits: torch.Tensor, out: torch.Tensor | None = None,
            keys: torch.Tensor | None = None) -> torch.Tensor:
-    """Greedy token of each row.  Long rows take two launches with a workspace
-    between them: `keys` (int64, argmax_num_keys elements), else one allocated
-    here.  With `out` and no `keys` the call allocates nothing, as a recorded
+    """Greedy token of each row.  A few long rows take two launches with a
+    workspace between them: `keys` (int64, argmax_num_keys elements), or above
+    ARGMAX_ALLOC_VOCAB one allocated here.  With `out` and no `keys` the call allocates nothing, as a recorded
     step must not, and the row takes one launch."""
     _check(logits, "logits", BF16)
     vocab = logits.shape[-1]
@@ -365,7 +376,7 @@ def argmax(logits: torch.Tensor, out: torch.Tensor | None = None,
     num_keys = argmax_num_keys(rows, vocab)
     if keys is not None:
         _check(keys, "keys", torch.int64, num_keys, logits.device)
-    elif num_keys and out is None:
+    elif num_keys and out is None and vocab > ARGMAX_ALLOC_VOCAB:
         keys = torch.empty((num_keys,), dtype=torch.int64, device=logits.device)
     if out is None:
         out = torch.empty((rows,), dtype=torch.int64, device=logits.device)

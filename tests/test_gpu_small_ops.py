@@ -192,7 +192,9 @@ def test_argmax(ops, dev):
 def test_argmax_edges(ops, dev, vocab, kind):
     """Rows that start 2 to 14 bytes past a 16-byte boundary, single elements
     around the chunks, zeros of both signs (equal), NaN of both signs (first
-    one wins), the lowest value everywhere."""
+    one wins), the lowest value everywhere; in one launch and, from 65536
+    elements on, in two."""
+    import torch
     rng = np.random.default_rng(vocab)
     x = randn_bf16(rng, (8, vocab))
     if kind == "zeros":
@@ -205,7 +207,27 @@ def test_argmax_edges(ops, dev, vocab, kind):
         x[:] = 0xFF80
     f = bf16_bits_to_f32(x)
     want = [int(np.argmax(np.isnan(r))) if np.isnan(r).any() else int(np.argmax(r)) for r in f]
-    assert ops.argmax(bf16_dev(x, dev)).cpu().tolist() == want
+    xd = bf16_dev(x, dev)
+    assert ops.argmax(xd).cpu().tolist() == want
+    keys = torch.empty(ops.argmax_num_keys(8, vocab), dtype=torch.int64, device=dev)
+    assert (keys.numel() > 0) == (vocab >= 65536)
+    assert ops.argmax(xd, keys=keys).cpu().tolist() == want
+
+
+@pytest.mark.parametrize("rows,vocab,keys,launch", [
+    (32, 65536, True, "parts"), (33, 65536, True, "one"), (1, 65535, True, "one"),
+    (1, 98304, False, "one"), (32, 98305, False, "parts"), (33, 98305, False, "one")])
+def test_argmax_launches(ops, dev, monkeypatch, rows, vocab, keys, launch):
+    import torch
+    x = torch.randn(rows, vocab, device=dev).to(torch.bfloat16)
+    k = (torch.empty(ops.argmax_num_keys(rows, vocab), dtype=torch.int64, device=dev) if keys
+         else None)
+    seen, real = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda name, *a: (seen.append(name), real(name, *a))[1])
+    got = ops.argmax(x, keys=k)
+    assert seen == [{"parts": "smx_argmax_bf16_parts", "one": "smx_argmax_bf16"}[launch]]
+    xc = x.cpu().float()
+    assert got.cpu().tolist() == [int((r == r.max()).nonzero()[0]) for r in xc]
 
 
 def test_argmax_ragged_vocab(ops, dev):
