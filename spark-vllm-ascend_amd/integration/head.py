@@ -4,8 +4,9 @@ Mirrors Q6HeadMethod (src/spark_vllm_ascend/integration/head.py:12-16,31):
 the head layer keeps its tied bf16 embedding weight, gains a packed
 quantized buffer, and its ``quant_method`` is swapped for a method whose
 ``apply`` serves bf16 input of 1 to 16 rows (batched decode) with the native
-kernels and defers to a plain bf16 matmul otherwise: more rows, a bias, or
-rows that torch has to see multiplied (linear.torch_sees).  The quantized head here is Q4_0
+kernels and defers to a plain bf16 matmul otherwise: more rows, a bias,
+tensors or blocks the batched kernel cannot read (gemm_takes), or a product
+that torch has to see (linear.torch_sees).  The quantized head here is Q4_0
 [vocab, hidden] (the reference model's head is Q6_K), and the tied
 embedding is bf16(dequantized head), the tying the reference prepares at
 src/tools/deployment/prepare_head.py:27.
@@ -27,12 +28,21 @@ class Q4_0HeadMethod:
             return torch_ops.q4_0_gemv(x.contiguous(), layer.q4_0_head, vocab, hidden)
         if (x.dim() == 2 and 2 <= x.shape[0] <= GEMM_MAX_ROWS and x.shape[1] == hidden
                 and x.dtype == torch.bfloat16 and bias is None and hidden % 64 == 0
-                and not layer.weight.requires_grad and not torch_sees(x)):
+                and gemm_takes(layer, x)
+                and not layer.weight.requires_grad and not torch_sees(x, layer.weight)):
             # a quarter of the bytes: 151936 x 2560 for 8 rows 69.5 us, 16 rows 116,
             # the bf16 product 242; 8000 x 512 3.3 and 7.6
             return torch_ops.q4_0_gemm(aligned16(x.contiguous()), layer.q4_0_head, vocab, hidden)
         out = torch.nn.functional.linear(x, layer.weight)
         return out if bias is None else out + bias
+
+
+def gemm_takes(layer: torch.nn.Module, x: torch.Tensor) -> bool:
+    """Whether q4_0_gemm can read x and the layer's blocks, and the bf16 product
+    it stands for would take x."""
+    w, blocks = layer.weight, layer.q4_0_head
+    return (x.is_cuda and w.device == x.device == blocks.device and w.dtype == x.dtype
+            and blocks.is_contiguous() and blocks.data_ptr() % 4 == 0)
 
 
 class TiedQ4_0Head(torch.nn.Module):

@@ -191,13 +191,13 @@ def aligned16(rows: torch.Tensor) -> torch.Tensor:
     return rows.clone() if rows.data_ptr() % 16 else rows
 
 
-def torch_sees(rows: torch.Tensor) -> bool:
-    """Whether a product of `rows` has to be a torch operation: autograd or a
-    forward-mode level records it, a functorch transform or a tensor subclass
+def torch_sees(*tensors: torch.Tensor) -> bool:
+    """Whether a product of the tensors has to be a torch operation: autograd or
+    a forward-mode level records it, a functorch transform or a tensor subclass
     or mode intercepts it, or autocast chooses its type."""
-    return (rows.requires_grad and torch.is_grad_enabled()
+    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
             or torch.is_autocast_enabled("cuda")
-            or type(rows) not in (torch.Tensor, torch.nn.Parameter)
+            or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors)
             or torch.autograd.forward_ad._current_level >= 0
             or torch._C._functorch.maybe_current_level() is not None
             or torch._C._len_torch_dispatch_stack() > 0

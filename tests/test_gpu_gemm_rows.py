@@ -144,6 +144,27 @@ def test_linear_routes(dev):
     assert torch.equal(layer(off[:5]), layer(x[:5]))
 
 
+@pytest.mark.parametrize("rows", [1, 2, 16])
+def test_head_blocks_of_any_alignment(dev, rows):
+    """Blocks 2 bytes past a 4-byte boundary, and blocks with a row stride (more
+    than one row), which the batched kernel does not read."""
+    import torch
+    head_mod = pkg("integration.head")
+    vocab, hidden = 1003, 320
+    blocks = oq.make_blocks(vocab, hidden, seed=9)
+    x = randn_bf16(np.random.default_rng(rows), (rows, hidden))
+    xd = bf16_dev(x, dev).view(rows, hidden)
+    head = head_mod.TiedQ4_0Head(_w(blocks, dev).view(vocab, -1), vocab, hidden)
+    row = blocks.size // vocab
+    wide = torch.zeros(vocab * row + 2, dtype=torch.uint8, device=dev)[2:].view(vocab, row)
+    strided = torch.zeros(vocab, row + 4, dtype=torch.uint8, device=dev)[:, :row]
+    for q in (wide, strided) if rows > 1 else (wide,):
+        q.copy_(_w(blocks, dev).view(vocab, row))
+        head.q4_0_head = q
+        y = f32_of(head.logits(xd)).reshape(rows, vocab)
+        _check(y, x, _weights(blocks, vocab, hidden, 1 if rows == 1 else 17))
+
+
 @pytest.mark.parametrize("rows", [2, 7, 16, 17])
 def test_head_rows(dev, rows):
     """2 to 16 rows of logits multiply the exact weights (any 2-D strides and

@@ -26,6 +26,26 @@ def test_plugin_import_is_stdlib_only():
     assert out.stdout.strip() == "", f"plugin import pulled in {out.stdout.strip()}"
 
 
+@pytest.mark.parametrize("device,rows", [("cpu", 2), ("cpu", 16), ("meta", 3)])
+def test_head_rows_off_the_gpu(device, rows):
+    """Several rows where the kernels cannot run are a bf16 product with the
+    tied weight; a weight of another type is refused as that product refuses it."""
+    import torch
+    head = pkg("integration.head")
+    layer = torch.nn.Module()
+    w = torch.randn(40, 64, dtype=torch.bfloat16, device=device)
+    layer.weight = torch.nn.Parameter(w, requires_grad=False)
+    layer.q4_0_head = torch.zeros(40, 36, dtype=torch.uint8, device=device)
+    x = torch.randn(rows, 64, dtype=torch.bfloat16, device=device)
+    y = head.Q4_0HeadMethod().apply(layer, x)
+    assert tuple(y.shape) == (rows, 40) and y.device.type == device
+    if device == "cpu":
+        assert torch.equal(y, torch.nn.functional.linear(x, w))
+        layer.weight = torch.nn.Parameter(w.float(), requires_grad=False)
+        with pytest.raises(RuntimeError):
+            head.Q4_0HeadMethod().apply(layer, x)
+
+
 def test_register_is_idempotent():
     plugin = pkg("plugin")
     a = plugin.register()
