@@ -28,13 +28,22 @@ class Q4_0HeadMethod:
             return torch_ops.q4_0_gemv(x.contiguous(), layer.q4_0_head, vocab, hidden)
         if (x.dim() == 2 and 2 <= x.shape[0] <= GEMM_MAX_ROWS and x.shape[1] == hidden
                 and x.dtype == torch.bfloat16 and bias is None and hidden % 64 == 0
-                and gemm_takes(layer, x)
+                and gemm_pays(x.shape[0], vocab, hidden) and gemm_takes(layer, x)
                 and not layer.weight.requires_grad and not torch_sees(x, layer.weight)):
-            # a quarter of the bytes: 151936 x 2560 for 8 rows 69.5 us, 16 rows 116,
-            # the bf16 product 242; 8000 x 512 3.3 and 7.6
             return torch_ops.q4_0_gemm(aligned16(x.contiguous()), layer.q4_0_head, vocab, hidden)
         out = torch.nn.functional.linear(x, layer.weight)
         return out if bias is None else out + bias
+
+
+def gemm_pays(rows: int, vocab: int, hidden: int) -> bool:
+    """Whether q4_0_gemm beats the bf16 product.  It reads a quarter of the
+    bytes (151936 x 2560: 8 rows 53 us, 16 rows 102, bf16 242; 8000 x 512 3.3 and
+    7.6), but above 8 rows its time grows faster with K, and a short bf16 product
+    is then the faster: 1000 x 8192 at 8 rows 6.8 against 8.3, at 9 rows 9.3; 16
+    rows of 32000 x 3072 32.4 against 31.6, 12 rows 29.0.
+    (Hidden sizes to 8192 measured above 8 rows.)"""
+    return (rows <= 8 or hidden <= 2560 or vocab >= 65536 and hidden <= 8192
+            or rows <= 12 and (hidden <= 5120 or vocab >= 4000 and hidden <= 8192))
 
 
 def gemm_takes(layer: torch.nn.Module, x: torch.Tensor) -> bool:

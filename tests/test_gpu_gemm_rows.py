@@ -144,6 +144,30 @@ def test_linear_routes(dev):
     assert torch.equal(layer(off[:5]), layer(x[:5]))
 
 
+@pytest.mark.parametrize("rows,vocab,hidden,fused", [
+    (8, 1000, 8192, True), (9, 1000, 8192, False), (12, 4000, 8192, True),
+    (13, 4000, 8192, False), (12, 1000, 5120, True), (13, 1000, 5120, False),
+    (16, 1000, 2560, True), (16, 65536, 4096, True), (17, 1000, 2560, False)])
+def test_head_launches(dev, monkeypatch, rows, vocab, hidden, fused):
+    """Which product each side of the line takes, both within their bounds."""
+    import torch
+    ops = pkg("native.torch_ops")
+    g = torch.Generator(device=dev)
+    g.manual_seed(rows)
+    q = torch.randint(0, 60, (vocab, hidden // 32 * 18), generator=g, dtype=torch.uint8, device=dev)
+    head = pkg("integration.head").TiedQ4_0Head(q, vocab, hidden)
+    x = torch.randn((rows, hidden), generator=g, device=dev).to(torch.bfloat16)
+    seen, real = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda name, *a: (seen.append(name), real(name, *a))[1])
+    y = head.logits(x).float()
+    assert seen == (["smx_q4_0_gemm"] if fused else [])
+    xd, wd = x.double().cpu(), head.weight[:500].double().cpu()
+    ref, mag = xd @ wd.T, xd.abs() @ wd.abs().T
+    # weights exact or rounded to bf16 (2^-9 of each product), fp32 sums, bf16 out
+    bound = 2.0 ** -8 * ref.abs() + (2.0 ** -9 + hidden * 2.0 ** -24) * mag
+    assert ((y[:, :500].cpu().double() - ref).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("rows", [1, 2, 16])
 def test_head_blocks_of_any_alignment(dev, rows):
     """Blocks 2 bytes past a 4-byte boundary, and blocks with a row stride (more
