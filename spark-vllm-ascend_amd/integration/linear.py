@@ -43,6 +43,15 @@ import torch
 from ..native import torch_ops
 from .weights import row_bytes
 
+try:
+    from torch._C import _len_torch_dispatch_stack, _len_torch_function_stack
+    from torch._C._functorch import maybe_current_level
+    from torch.overrides import _get_current_function_mode_stack
+    from torch.utils._device import DeviceContext
+    _STATE_KNOWN = isinstance(torch.autograd.forward_ad._current_level, int)
+except (ImportError, AttributeError):  # another torch: torch_sees() is always true
+    _STATE_KNOWN = False
+
 try:  # pragma: no cover - vLLM is absent here
     from vllm.model_executor.layers.linear import LinearMethodBase as _Base
 except Exception:  # noqa: BLE001
@@ -195,13 +204,16 @@ def torch_sees(*tensors: torch.Tensor) -> bool:
     """Whether a product of the tensors has to be a torch operation: autograd or
     a forward-mode level records it, a functorch transform or a tensor subclass
     or mode intercepts it, or autocast chooses its type."""
-    return (torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
+    return (not _STATE_KNOWN
+            or torch.is_grad_enabled() and any(t.requires_grad for t in tensors)
             or torch.is_autocast_enabled("cuda")
             or any(type(t) not in (torch.Tensor, torch.nn.Parameter) for t in tensors)
             or torch.autograd.forward_ad._current_level >= 0
-            or torch._C._functorch.maybe_current_level() is not None
-            or torch._C._len_torch_dispatch_stack() > 0
-            or torch._C._len_torch_function_stack() > 0)
+            or maybe_current_level() is not None
+            or _len_torch_dispatch_stack() > 0
+            # a default device is a mode too, one that leaves products alone
+            or _len_torch_function_stack() > 0 and not all(
+                isinstance(m, DeviceContext) for m in _get_current_function_mode_stack()))
 
 
 def gemm_weight(layer: torch.nn.Module, gated: bool = False):

@@ -144,6 +144,59 @@ def test_linear_routes(dev):
     assert torch.equal(layer(off[:5]), layer(x[:5]))
 
 
+@pytest.mark.parametrize("state", ["plain", "no_grad", "default device", "autograd", "vmap",
+                                   "forward mode", "autocast", "function mode"])
+def test_linear_launches(dev, monkeypatch, state):
+    """One launch for rows that torch only multiplies, a default device set or
+    not; dequantisation and torch's product where torch has to see it."""
+    import torch
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    ops = pkg("native.torch_ops")
+    n, k, m = 4001, 2592, 40
+    layer = pkg("integration.linear").Q4_0Linear(k, [n], device=dev)
+    layer.qweight.data.copy_(_w(oq.make_blocks(n, k, seed=5), dev).view(n, -1))
+    x = bf16_dev(randn_bf16(np.random.default_rng(6), (m, k)), dev).view(m, k)
+    want = layer(x).float()
+    seen, real = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda name, *a: (seen.append(name), real(name, *a))[1])
+
+    class Mode(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    if state == "plain":
+        y = layer(x)
+    elif state == "no_grad":
+        with torch.no_grad():
+            y = layer(x.clone().requires_grad_(True))
+    elif state == "default device":
+        with torch.device(dev):
+            y = layer(x)
+    elif state == "autograd":
+        y = layer(x.clone().requires_grad_(True)).detach()
+    elif state == "vmap":
+        y = torch.func.vmap(layer)(torch.stack((x, x)))[1]
+    elif state == "forward mode":
+        with forward_ad.dual_level():
+            d = forward_ad.unpack_dual(layer(forward_ad.make_dual(x, x)))
+            assert torch.equal(d.primal, d.tangent)
+            y = d.primal
+    elif state == "autocast":
+        with torch.autocast("cuda", dtype=torch.float16):
+            y = layer(x)
+        assert y.dtype == torch.float16
+    else:
+        with Mode():
+            y = layer(x)
+    fused = state in ("plain", "no_grad", "default device")
+    assert seen == ["smx_q4_0_gemm_rows" if fused else "smx_q4_0_dequant_bf16"]
+    torch.testing.assert_close(y.float(), want, rtol=2.0 ** -6, atol=1e-2)
+    seen.clear()
+    layer(x[:5])
+    assert seen == ["smx_q4_0_gemm_rows"]
+
+
 @pytest.mark.parametrize("rows,vocab,hidden,fused", [
     (8, 1000, 8192, True), (9, 1000, 8192, False), (12, 4000, 8192, True),
     (13, 4000, 8192, False), (12, 1000, 5120, True), (13, 1000, 5120, False),

@@ -46,6 +46,60 @@ def test_head_rows_off_the_gpu(device, rows):
             head.Q4_0HeadMethod().apply(layer, x)
 
 
+def test_torch_sees():
+    """Which states keep a product a torch operation (CPU: it reads torch's
+    state alone)."""
+    import torch
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+    sees = pkg("integration.linear").torch_sees
+    x, w = torch.ones(2, 3), torch.nn.Parameter(torch.ones(4, 3), requires_grad=False)
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    assert not sees(x) and not sees(x, w)
+    g = x.clone().requires_grad_(True)
+    assert sees(g) and sees(x, torch.nn.Parameter(w.data))
+    with torch.no_grad():
+        assert not sees(g)
+    assert sees(x.as_subclass(Sub)) and sees(x, w.data.as_subclass(Sub))
+    seen = []
+    torch.func.vmap(lambda r: (seen.append(sees(r)), r)[1])(x)
+    torch.func.grad(lambda r: (seen.append(sees(r)), r.sum())[1])(x)
+    with forward_ad.dual_level():
+        seen.append(sees(x))
+    with Function():
+        seen.append(sees(x))
+    with Dispatch():
+        seen.append(sees(x))
+    torch.set_autocast_enabled("cuda", True)
+    seen.append(sees(x))
+    torch.set_autocast_enabled("cuda", False)
+    with torch.device("cpu"), Function():
+        seen.append(sees(x))
+    assert seen == [True] * 7
+    # a default device changes no product
+    with torch.device("cpu"):
+        assert not sees(x)
+    old = torch.get_default_device()
+    torch.set_default_device("cpu")
+    try:
+        assert not sees(x)
+    finally:
+        torch.set_default_device(None if old == torch.device("cpu") else old)
+    assert not sees(x)
+
+
 def test_register_is_idempotent():
     plugin = pkg("plugin")
     a = plugin.register()
