@@ -405,17 +405,27 @@ extern "C" int smx_q4_0_gemm_rows(void* stream, const void* x, const void* w, vo
 
 // 1 where the fused kernel is the faster way to an [m, n] product with bf16
 // weight roundings (m > 16), 0 where dequantising the matrix and multiplying
-// with a library GEMM is.  Measured for that way (us, 64 / 193 / 256 rows):
-// 6144 x 2560 29.7 / 32.9 / 40.3, 9728 x 2560 32.8 / 40.2 / 44.8, 19456 x 2560
-// 44.6 / 59.9 / 60.6, 2560 x 9728 39.4 / 45.3 / 44.4, 4001 x 2592 27.6 / 31.5 /
-// 31.6: about 22 + (0.3 + 0.0025 m) per million weights.  It grows slower than
-// the fused kernel's time, which pays for the conversion once per row group:
-// 512 rows of 9728 x 2560 are 47.9 against 62.9.
+// with a library GEMM is.  That way grows slower with m, as the fused kernel
+// pays for the conversion once per row group.  Its estimate is a fit to both
+// ways measured at 18 row counts of 61 sizes: a launch and a half, the matrix
+// written and read back (dearer once its bf16 form leaves the last-level cache
+// at 100 million weights), less for the outputs a short K has many of.  Of the
+// 793 sizes it picks the fused kernel for, 5 are slower by it, at most 12 %
+// (22016 x 4096 at 128 rows 77.7 us against 69.6; 19456 x 2560 at 128 rows 50.8,
+// 48.4); of 244 at 16 sizes it was not fitted to, 6, at most 6 %.  us, fused and
+// library:
+//   6144 x 2560    48 rows 12.4, 29.9   256 rows 29.2, 40.2   512 rows 37.2, 36.0
+//   9728 x 2560    64 rows 18.5, 32.8   193 rows 33.1, 39.5   512 rows 62.9, 47.9
+//   19456 x 2560   96 rows 35.1, 46.4   256 rows 67.3, 59.5
+//   2560 x 4096   128 rows 14.9, 32.3   320 rows 26.3, 27.7   512 rows 34.8, 29.3
+//   20000 x 160    64 rows  8.7, 12.1   256 rows 20.9, 17.3
 extern "C" int smx_q4_0_gemm_rows_preferred(int64_t m, int64_t n, int64_t k) {
   if (m < 17 || m > 512 || n < 1 || n > (1ll << 30) || k < 32 || k % 32 != 0 ||
       k > (1 << 20) || m * k >= (1ll << 30))
     return 0;
   float fused;
   smx::rows_pick(m, n, k / 32, &fused);
-  return fused < 22.0f + 1e-6f * (float)n * (float)k * (0.3f + 0.0025f * (float)m);
+  const float mw = 1e-6f * (float)n * (float)k, mo = 1e-6f * (float)m * (float)n;
+  return fused < 15.2f + 0.86f * fminf(mw, 12.0f) + mw * (0.7f + 0.0003f * (float)m) +
+                     0.6f * fmaxf(mw - 100.0f, 0.0f) - 2.2f * mo;
 }

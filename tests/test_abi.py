@@ -125,6 +125,17 @@ def test_invalid_arguments_rejected_on_host(call, args):
     assert lib.smx_last_error().decode().startswith(call)
 
 
+@pytest.mark.parametrize("m,n,k,fused", [
+    (48, 6144, 2560, 1), (193, 9728, 2560, 1), (40, 4001, 2592, 1), (112, 19456, 2560, 1),
+    (320, 2560, 4096, 1), (64, 151936, 2560, 1), (300, 1024, 16384, 1), (96, 20000, 160, 1),
+    (512, 6144, 2560, 0), (256, 19456, 2560, 0), (400, 2560, 4096, 0), (512, 4096, 4096, 0),
+    (256, 20000, 160, 0), (384, 16384, 1024, 0), (512, 5120, 5120, 0), (193, 49152, 256, 0),
+    (16, 6144, 2560, 0), (513, 512, 8192, 0), (64, 512, 48, 0), (512, 64, 1 << 21, 0)])
+def test_rows_gemm_rule(m, n, k, fused):
+    """The side measured as the faster one, and the sizes outside its range."""
+    assert pkg("native").load().smx_q4_0_gemm_rows_preferred(m, n, k) == fused
+
+
 def test_argmax_keys_size():
     native = pkg("native")
     lib = native.load()
