@@ -75,6 +75,12 @@ GEMM_MAX_ROWS = 16
 #: the host's (1024 x 2560 at 40 rows: 14.6 us, fused 6.4)
 GEMM_ROWS_MIN_WEIGHTS = 3_000_000
 
+#: K up to which 2 and 3 rows of a matrix of few rows (n < 1536) are one
+#: q4_0_gemm_rows launch.  Its 8 waves walk K, 0.7 us per 1024, where a GEMV splits
+#: it further: 300 x 10016 at 2 rows 10.5 us, two GEMVs 10.9; 96 x 32800 27.1,
+#: 20.2; at 3 rows 27.1, 29.8; 48 x 65568 49.9, 49.4; 4 rows 49.9, 65.4
+FEW_ROWS_MAX_K = {2: 10240, 3: 40960}
+
 
 class Q4_0Config:
     """Quantization config naming the method, as vLLM's QuantizationConfig.
@@ -163,7 +169,8 @@ class Q4_0LinearMethod(_Base):
             out = torch_ops.q4_0_gemv(rows, w, n, k)
         elif m <= GEMM_MAX_ROWS and k % 64 == 0:
             out = torch_ops.q4_0_gemm(aligned16(rows), gemm_weight(layer), n, k)
-        elif m <= GEMM_MAX_ROWS and n * k >= GEMM_ROWS_MIN_WEIGHTS and w.data_ptr() % 4 == 0:
+        elif (m <= GEMM_MAX_ROWS and n * k >= GEMM_ROWS_MIN_WEIGHTS and w.data_ptr() % 4 == 0
+              and (n >= 1536 or k <= FEW_ROWS_MAX_K.get(m, k))):
             # K % 64 != 0: one launch for all rows (4001 x 2592, 5 rows: 5.5 us;
             # the GEMV below is 5.8 us for each)
             out = torch_ops.q4_0_gemm_rows(aligned16(rows), w, n, k)

@@ -144,6 +144,23 @@ def test_linear_routes(dev):
     assert torch.equal(layer(off[:5]), layer(x[:5]))
 
 
+@pytest.mark.parametrize("m,n,k,fused", [
+    (2, 300, 10016, True), (2, 300, 10272, False), (2, 1536, 10272, True),
+    (3, 96, 40928, True), (3, 96, 41056, False), (4, 96, 41056, True)])
+def test_linear_few_rows_launches(dev, monkeypatch, m, n, k, fused):
+    """One launch or a GEMV per row where K % 64 != 0, on both sides of the line."""
+    ops = pkg("native.torch_ops")
+    layer = pkg("integration.linear").Q4_0Linear(k, [n], device=dev)
+    blocks = oq.make_blocks(n, k, seed=n + m)
+    layer.qweight.data.copy_(_w(blocks, dev).view(n, -1))
+    x = randn_bf16(np.random.default_rng(m), (m, k))
+    seen, real = [], ops.call
+    monkeypatch.setattr(ops, "call", lambda name, *a: (seen.append(name), real(name, *a))[1])
+    y = f32_of(layer(bf16_dev(x, dev).view(m, k))).reshape(m, n)
+    assert seen == (["smx_q4_0_gemm_rows"] if fused else ["smx_q4_0_gemv"] * m)
+    _check(y, x, _weights(blocks, n, k, m))
+
+
 @pytest.mark.parametrize("state", ["plain", "no_grad", "default device", "autograd", "vmap",
                                    "forward mode", "autocast", "function mode"])
 def test_linear_launches(dev, monkeypatch, state):
