@@ -144,10 +144,17 @@ __global__ __launch_bounds__(64) void qknorm_rope_kv_kernel(
 
 // The same with 16-byte accesses (every tensor 16-byte aligned): 16 lanes per
 // head, lane j dims 8 j .. 8 j + 7, four consecutive (token, head) pairs per
-// wave.  Bound by memory; a wave per head with 2-byte accesses moved a
-// prefill chunk of 2047 tokens x 48 heads in 25.9 us, this in 13.6 (50 MB).  Lane j ^ 8
+// wave.  A wave per head with 2-byte accesses moved a prefill chunk of 2047
+// tokens x 48 heads in 25.9 us, this in 13.6: 50 MB at 3.7 TB/s, short of what a
+// copy streams, as each lane has one load of its own in flight and then the
+// chain of position, rotary row and the lane moves.  Lane j ^ 8
 // holds the other half of each rotation pair and the squares are summed in
-// the one-wave kernel's order, so both kernels round alike.
+// the one-wave kernel's order, so both kernels round alike.  Below
+// QKNORM_VEC_ITEMS pairs a wave per head is the faster, its chain being shorter
+// (48 heads: 1 token 2.45 us, this 2.66; 16 tokens 2.60, 2.74; 24 both 2.78; 48
+// 3.07, 2.79).
+constexpr uint32_t QKNORM_VEC_ITEMS = 1536;
+
 __global__ __launch_bounds__(256) void qknorm_rope_kv_vec_kernel(
     const uint16_t* __restrict__ qkv, const uint16_t* __restrict__ q_gamma,
     const uint16_t* __restrict__ k_gamma, const uint16_t* __restrict__ cos_sin,
@@ -673,8 +680,9 @@ extern "C" int smx_qknorm_rope_kv_write(void* stream, const void* qkv, const voi
   SMX_REQUIRE(eps >= 0.f && isfinite(eps), "eps must be finite and >= 0");
   SMX_REQUIRE((uintptr_t)positions % 8 == 0 && (uintptr_t)slot_mapping % 8 == 0,
               "int64 arrays must be 8-byte aligned");
-  if (aligned16(qkv, q_gamma, k_gamma, cos_sin, q_out, k_cache, v_cache)) {
-    const uint32_t items = (uint32_t)num_tokens * (uint32_t)(n_q + 2 * n_kv);  // <= 65535^2
+  const uint32_t items = (uint32_t)num_tokens * (uint32_t)(n_q + 2 * n_kv);  // <= 65535^2
+  if (items >= smx::QKNORM_VEC_ITEMS &&
+      aligned16(qkv, q_gamma, k_gamma, cos_sin, q_out, k_cache, v_cache)) {
     SMX_LAUNCH(smx::qknorm_rope_kv_vec_kernel, dim3(items / 16 + (items % 16 != 0)), dim3(256), 0,
                (hipStream_t)stream, (const uint16_t*)qkv, (const uint16_t*)q_gamma,
                (const uint16_t*)k_gamma, (const uint16_t*)cos_sin, positions, slot_mapping,
@@ -705,13 +713,22 @@ int launch_gated_vec(void* stream, const void* gate_up, const void* lut, void* o
 }
 }  // namespace
 
+// Whether a gated activation takes the kernel with 16-byte accesses.  The line:
+// from there on it beats one element a thread (us, element-wise and this: SiLU
+// 131072 outputs 2.38, 2.49; 233472 2.60, 2.53; 622592 3.19, 2.87.  GELU, which
+// fills its table first: 131072 2.59, 3.66; 622592 3.58, 3.91; 933888 4.33, 3.99).
+static bool gated_vec(bool gelu, const void* gate_up, const void* out, int64_t rows, int64_t d) {
+  return d % 8 == 0 && rows * d >= (gelu ? 7 << 17 : 1 << 18) && rows * d < (1ll << 34) &&
+         aligned16(gate_up, out);
+}
+
 extern "C" int smx_silu_mul(void* stream, const void* gate_up, void* out, int64_t rows,
                             int64_t d) {
   SMX_REQUIRE(gate_up && out, "null pointer argument");
   SMX_REQUIRE(rows >= 1 && d >= 1 && rows * d < (1ll << 40), "bad shape");
   const int64_t grid = (rows * d + 255) / 256;
   SMX_REQUIRE(grid < (1ll << 31), "tensor too large");
-  if (d % 8 == 0 && rows * d < (1ll << 34) && aligned16(gate_up, out))
+  if (gated_vec(false, gate_up, out, rows, d))
     return launch_gated_vec<false>(stream, gate_up, nullptr, out, rows, d);
   SMX_LAUNCH(smx::silu_mul_kernel, dim3((unsigned)grid), dim3(256), 0,
                      (hipStream_t)stream, (const uint16_t*)gate_up, (uint16_t*)out, rows, d);
@@ -726,7 +743,7 @@ extern "C" int smx_gelu_mul(void* stream, const void* gate_up, const void* lut, 
   SMX_REQUIRE(rows >= 1 && d >= 1 && rows * d < (1ll << 40), "bad shape");
   const int64_t grid = (rows * d + 255) / 256;
   SMX_REQUIRE(grid < (1ll << 31), "tensor too large");
-  if (d % 8 == 0 && rows * d < (1ll << 34) && aligned16(gate_up, out))
+  if (gated_vec(true, gate_up, out, rows, d))
     return launch_gated_vec<true>(stream, gate_up, lut, out, rows, d);
   SMX_LAUNCH(smx::gelu_mul_kernel, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream,
              (const uint16_t*)gate_up, (const uint16_t*)lut, (uint16_t*)out, rows, d);

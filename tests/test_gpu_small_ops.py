@@ -103,11 +103,14 @@ def _off(t, shift):
     return buf[shift:].view(t.shape)
 
 
-@pytest.mark.parametrize("rows,d", [(1, 8), (3, 40), (63, 2056), (2, 9728), (257, 8200)])
+@pytest.mark.parametrize("rows,d", [(1, 8), (3, 40), (63, 2056), (2, 9728), (257, 8200),
+                                    (33, 8200), (113, 8200), (114689, 8)])
 @pytest.mark.parametrize("act", ["silu", "gelu"])
 def test_gated_vector_kernel_equals_scalar(ops, dev, rows, d, act):
     """16-byte and element-wise kernels, bit for bit: sizes around a
-    workgroup's chunks, one and four chunks a thread; nothing past the end."""
+    workgroup's chunks, one and four chunks a thread, and sizes that stay with
+    the element-wise kernel (below 2^18 outputs for SiLU and 7 * 2^17 for GELU,
+    whatever the alignment); nothing past the end."""
     import torch
     gu = torch.randn(rows, 2 * d, device=dev).mul_(4).to(torch.bfloat16)
     gu[0, 0], gu[-1, d - 1] = float("inf"), float("-inf")
@@ -121,10 +124,12 @@ def test_gated_vector_kernel_equals_scalar(ops, dev, rows, d, act):
     assert bool((buf[rows * d:] == -7.0).all())
 
 
-@pytest.mark.parametrize("T,n_q,n_kv", [(1, 4, 1), (5, 3, 1), (17, 32, 8), (3, 8, 2)])
+@pytest.mark.parametrize("T,n_q,n_kv", [(1, 4, 1), (5, 3, 1), (17, 32, 8), (3, 8, 2),
+                                        (307, 3, 1), (308, 3, 1), (32, 32, 8), (129, 8, 2)])
 def test_qknorm_vector_kernel_equals_scalar(ops, dev, T, n_q, n_kv):
     """The 16-lanes-a-head kernel against the wave-a-head one, bit for bit,
-    with head counts that leave a partial wave and slots that are skipped."""
+    with head counts that leave a partial wave and slots that are skipped, on
+    both sides of the 1536 heads from which the first is taken."""
     import torch
     torch.manual_seed(T)
     nh = n_q + 2 * n_kv
@@ -132,11 +137,12 @@ def test_qknorm_vector_kernel_equals_scalar(ops, dev, T, n_q, n_kv):
     qg, kg = ((1 + 0.1 * torch.randn(128, device=dev)).to(torch.bfloat16) for _ in range(2))
     cs = torch.randn(64, 128, device=dev).to(torch.bfloat16)
     pos = torch.randint(-2, 70, (T,), device=dev)  # clamped to the table
-    slots = torch.randperm(96, device=dev)[:T].clone()
+    blocks = max(3, T // 32 + 2)
+    slots = torch.randperm(32 * blocks, device=dev)[:T].clone()
     slots[T // 2] = -1 if T > 1 else slots[0]
     res = []
     for shift in (0, 1):
-        kv = torch.zeros(2, 3, 32, n_kv, 128, dtype=torch.bfloat16, device=dev)
+        kv = torch.zeros(2, blocks, 32, n_kv, 128, dtype=torch.bfloat16, device=dev)
         q = ops.qknorm_rope_kv_write(_off(qkv, shift), qg, kg, cs, pos, slots, kv[0], kv[1], n_q,
                                      n_kv, 1e-6)
         res.append((bits_of(q), bits_of(kv)))
