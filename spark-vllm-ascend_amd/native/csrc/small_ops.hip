@@ -681,7 +681,8 @@ extern "C" int smx_qknorm_rope_kv_write(void* stream, const void* qkv, const voi
   SMX_REQUIRE((uintptr_t)positions % 8 == 0 && (uintptr_t)slot_mapping % 8 == 0,
               "int64 arrays must be 8-byte aligned");
   const uint32_t items = (uint32_t)num_tokens * (uint32_t)(n_q + 2 * n_kv);  // <= 65535^2
-  if (items >= smx::QKNORM_VEC_ITEMS &&
+  // (a grid dimension holds fewer than 2^32 work-items: 16 a pair here)
+  if (items >= smx::QKNORM_VEC_ITEMS && items < (1u << 28) &&
       aligned16(qkv, q_gamma, k_gamma, cos_sin, q_out, k_cache, v_cache)) {
     SMX_LAUNCH(smx::qknorm_rope_kv_vec_kernel, dim3(items / 16 + (items % 16 != 0)), dim3(256), 0,
                (hipStream_t)stream, (const uint16_t*)qkv, (const uint16_t*)q_gamma,

@@ -136,6 +136,21 @@ def test_runner_records_argmax_with_its_outputs(dev):
         ops.argmax(logits, out=out, keys=keys[1:])
 
 
+@pytest.mark.parametrize("n_kv", [2047, 2048])
+def test_recorded_qknorm_grid_of_any_size(dev, n_kv):
+    """65535 tokens of 4095 and 4097 heads, just below and above 2^28 pairs: a
+    launch shape of fewer than 2^32 work-items a dimension (recorded only: the
+    pointers are never read)."""
+    import torch
+    ops = pkg("native.torch_ops")
+    b = torch.zeros(256, dtype=torch.bfloat16, device=dev)
+    p, i = b.data_ptr(), torch.zeros(4, dtype=torch.int64, device=dev).data_ptr()
+    with pkg("native.runner").StepRunner() as runner:
+        assert runner.record(lambda: ops.call(
+            "smx_qknorm_rope_kv_write", torch.cuda.current_stream().cuda_stream, p, p, p, p, i, i,
+            p, p, p, 65535, 1, n_kv, 128, 1, 32, 1, 1e-6)) == 1
+
+
 @pytest.mark.parametrize("fences", FENCES)
 def test_runner_steps_per_call_do_not_matter(dev, fences):
     _eager_vs_runner(dev, fences, chunks=(1, 1, 5, 23), seed=6)
