@@ -171,22 +171,6 @@ __global__ __launch_bounds__(512) void q4_0_gemm_kernel(GemmArgs a) {
 // The waves of a workgroup take the tiles t = wave, wave + ks, ...
 // ---------------------------------------------------------------------------
 
-// 4x4 transpose across the four 16-lane rows: on entry row j of r_g holds
-// X[j][g]; on exit row g of r_k holds X[k][g].  v_permlane16_swap(a, b)
-// swaps the odd rows of a with the even rows of b; v_permlane32_swap(a, b)
-// swaps rows 2-3 of a with rows 0-1 of b.
-__device__ __forceinline__ void transpose_rows4(uint32_t& r0, uint32_t& r1, uint32_t& r2,
-                                                uint32_t& r3) {
-  const auto a = __builtin_amdgcn_permlane16_swap(r0, r1, false, false);
-  const auto b = __builtin_amdgcn_permlane16_swap(r2, r3, false, false);
-  const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
-  const auto d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
-  r0 = c[0];
-  r2 = c[1];
-  r1 = d[0];
-  r3 = d[1];
-}
-
 // WS > 0 (m <= 2 WS <= 8): a wave copies its tile's activations -- m rows x
 // 512 bytes, WS 16-byte loads per lane -- into a private LDS slice and reads
 // the MFMA A operands from there (8 loads per tile straight from global

@@ -74,8 +74,7 @@ __device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0); }
 // Unaligned-to-16 (but 4-byte aligned) vector types for the Q4_0 stream:
 // GGUF blocks are 18 bytes, so a block pair starts on a 4-byte boundary only.
 typedef u32x4 u32x4_a4 __attribute__((aligned(4)));
-typedef u32x4 u32x4_a2 __attribute__((aligned(2)));  // one block of a row of any K % 32
-typedef u32x2 u32x2_a2 __attribute__((aligned(2)));
+typedef u32x2 u32x2_a2 __attribute__((aligned(2)));  // half a block of any row
 
 __device__ __forceinline__ float bf16_bits_to_f32(uint32_t h16) {
   return __uint_as_float(h16 << 16);
@@ -156,6 +155,22 @@ constexpr int DPP_QUAD_XOR2 = 0x4E;      // quad_perm [2,3,0,1]
 constexpr int DPP_ROW_HALF_MIRROR = 0x141;
 constexpr int DPP_ROW_MIRROR = 0x140;
 constexpr int DPP_ROW_ROR8 = 0x128;      // lane j of a row gets lane j ^ 8
+
+// 4x4 transpose across the four 16-lane rows: on entry row j of r_g holds
+// X[j][g]; on exit row g of r_k holds X[k][g].  v_permlane16_swap(a, b)
+// swaps the odd rows of a with the even rows of b; v_permlane32_swap(a, b)
+// swaps rows 2-3 of a with rows 0-1 of b.
+__device__ __forceinline__ void transpose_rows4(uint32_t& r0, uint32_t& r1, uint32_t& r2,
+                                                uint32_t& r3) {
+  const auto a = __builtin_amdgcn_permlane16_swap(r0, r1, false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(r2, r3, false, false);
+  const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  r0 = c[0];
+  r2 = c[1];
+  r1 = d[0];
+  r3 = d[1];
+}
 
 // Sum over each aligned group of 8 lanes; every lane of the group gets it.
 __device__ __forceinline__ float sum8(float v) {
