@@ -122,9 +122,56 @@ def test_rows_infinities(ops, dev):
         np.testing.assert_array_equal(np.isposinf(y), np.isposinf(ref[:rows]))
 
 
+@pytest.mark.parametrize("m", [16, 40])
+def test_rows_subnormal_scales_bits(ops, dev, m):
+    """One-hot activations select weights of subnormal and extreme finite
+    scales of both signs bit for bit (zeros by value)."""
+    n, k = 48, 416
+    blocks = oq.make_blocks(n, k, seed=21)
+    scales = np.uint16([0x0001, 0x8001, 0x03FF, 0x83FF, 0x0400, 0x7BFF, 0xFBFF, 0x0000, 0x8000])
+    view = blocks.reshape(n * k // 32, 18)
+    view[:, :2] = scales[np.arange(len(view)) % len(scales)][:, None].view(np.uint8)
+    cols = (np.arange(m) * 37 + 5) % k
+    x = np.zeros((m, k), dtype=np.uint16)
+    x[np.arange(m), cols] = 0x3F80
+    y = ops.q4_0_gemm_rows(bf16_dev(x, dev), _w(blocks, dev), n, k)
+    want = f32_to_bf16_bits(oq.dequant_f32(blocks, n, k).reshape(n, k)[:, cols].T + np.float32(0))
+    np.testing.assert_array_equal(f32_of(y).reshape(m, n), bf16_bits_to_f32(want))
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 40])
+def test_rows_infinite_and_nan_scales(ops, dev, m):
+    """Infinite and NaN scales: above 16 rows what a product with the
+    dequantised weights gives, up to 16 what the GEMV gives a row (the scale
+    times a block's sum); rows without one keep their bounds."""
+    n, k = 50, 288
+    blocks = oq.make_blocks(n, k, seed=22)
+    view = blocks.reshape(n, k // 32, 18)
+    for r, b, h in ((3, 0, 0x7C00), (7, 4, 0xFC00), (20, 8, 0x7E00), (49, 8, 0x7C00)):
+        view[r, b, :2] = np.uint16([h]).view(np.uint8)
+    special = np.isin(np.arange(n), (3, 7, 20, 49))
+    x = randn_bf16(np.random.default_rng(m), (m, k))
+    xd, wd = bf16_dev(x, dev).view(m, k), _w(blocks, dev)
+    y = f32_of(ops.q4_0_gemm_rows(xd, wd, n, k)).reshape(m, n)
+    if m <= 16:
+        ref = np.stack([f32_of(ops.q4_0_gemv(xd[r], wd, n, k)).reshape(n) for r in range(m)])
+    else:
+        w = f32_of(ops.q4_0_dequant_bf16(wd, n, k)).reshape(n, k).astype(np.float64)
+        with np.errstate(invalid="ignore"):
+            ref = bf16_bits_to_f32(x).astype(np.float64) @ w.T
+    assert not np.isfinite(ref[:, special]).any() and np.isfinite(ref[:, ~special]).all()
+    np.testing.assert_array_equal(np.isnan(y), np.isnan(ref))
+    np.testing.assert_array_equal(np.isposinf(y), np.isposinf(ref))
+    np.testing.assert_array_equal(np.isneginf(y), np.isneginf(ref))
+    with np.errstate(invalid="ignore"):
+        w = _weights(blocks, n, k, m)
+    _check(y[:, ~special], x, w[~special])
+
+
 def test_linear_routes(dev):
-    """Rows that torch only multiplies take the fused kernel, rows that
-    autograd records keep the library product and its gradient."""
+    """Rows that autograd records keep the library product and its gradient,
+    and rows of any alignment give the same result (which launch each state
+    makes: test_linear_launches)."""
     import torch
     lin = pkg("integration.linear")
     n, k, m = 4001, 2592, 40
