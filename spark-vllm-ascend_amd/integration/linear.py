@@ -69,10 +69,11 @@ except Exception:  # noqa: BLE001
 #: activation rows one MFMA Q4_0 GEMM launch serves (the kernel's m limit)
 GEMM_MAX_ROWS = 16
 
-#: weights (n * k) from which q4_0_gemm_rows takes a call.  Smaller matrices
-#: keep the launches that callers and the boundary tests know for them (the GEMV
-#: per row, dequantisation and the library), where the device's time hides behind
-#: the host's (1024 x 2560 at 40 rows: 14.6 us, fused 6.4)
+#: weights (n * k) from which q4_0_gemm_rows takes a call.  Not a crossover: smaller
+#: matrices keep the launches that the dispatch tests fix for them (the GEMV per
+#: row, dequantisation and the library), although one launch is the faster there
+#: too (eager, kept and fused: 1024 x 2560 at 40 rows 28 us and 11, 512 x 2592 at
+#: 3 rows 22 and 10)
 GEMM_ROWS_MIN_WEIGHTS = 3_000_000
 
 #: K up to which 2 and 3 rows of a matrix of few rows (n < 1536) are one
