@@ -136,6 +136,27 @@ def test_runner_records_argmax_with_its_outputs(dev):
         ops.argmax(logits, out=out, keys=keys[1:])
 
 
+@pytest.mark.parametrize("m,n,k", [(5, 4001, 2592), (48, 6144, 2560), (193, 9728, 2560)])
+def test_runner_records_the_row_gemm(dev, m, n, k):
+    """Its launches take up to 80 KB of dynamic LDS here: recorded and replayed
+    on new activations, bit for bit what the direct call gives."""
+    import torch
+    ops = pkg("native.torch_ops")
+    g = torch.Generator(device=dev)
+    g.manual_seed(m)
+    w = torch.randint(0, 60, (n * k // 32 * 18,), generator=g, dtype=torch.uint8, device=dev)
+    x = torch.randn((m, k), generator=g, device=dev).to(torch.bfloat16)
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=dev)
+    with pkg("native.runner").StepRunner() as runner:
+        assert runner.record(lambda: ops.q4_0_gemm_rows(x, w, n, k, out=out)) == 1
+        for _ in range(2):
+            x.copy_(torch.randn((m, k), generator=g, device=dev))
+            out.zero_()
+            runner.run(1)
+            got = out.clone()
+            np.testing.assert_array_equal(bits_of(got), bits_of(ops.q4_0_gemm_rows(x, w, n, k)))
+
+
 @pytest.mark.parametrize("n_kv", [2047, 2048])
 def test_recorded_qknorm_grid_of_any_size(dev, n_kv):
     """65535 tokens of 4095 and 4097 heads, just below and above 2^28 pairs: a
